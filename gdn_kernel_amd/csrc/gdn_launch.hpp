@@ -47,7 +47,7 @@ struct PrefillArgs {
   // Two-kernel path: workspace of prefill_workspace_bytes(...) bytes for the
   // prepared T~/P tiles; null (or a batch that the single kernel serves) => one kernel.
   uint16_t* tiles;
-  int prep_chunks;          // set by the launcher: consecutive chunks per prep workgroup
+  int prep_slots;           // set by the launcher: most chunks of a batch with valid offsets
 };
 
 // Workspace bytes of the two-kernel prefill path for these sizes on the current

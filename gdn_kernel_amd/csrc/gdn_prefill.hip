@@ -93,7 +93,6 @@ template <int NCW_, int VT_, bool HOOKS_ = false, bool LOAD_ = false, int NP_ = 
 struct Variant {
   static constexpr bool kHooks = HOOKS_;         // testing hooks of PrefillArgs compiled in
   static constexpr bool kLoad = LOAD_;           // waves NCW.. load prepared T~/P (two-kernel path)
-  static constexpr bool kCopy = false;           // producers copy their tiles out (prep kernel only)
   static constexpr int NCW = NCW_;               // consumer waves
   static constexpr int NP = NP_;                 // producer (or loader) waves: 4; or 7 (6) beside one (two) consumers
   static constexpr int VT = VT_;                 // 16-row state tiles per consumer wave
@@ -139,40 +138,28 @@ using SplitVariant8 = Variant<1, 1, HOOKS, false, 7>;
 template <bool HOOKS>
 using PersistVariant = Variant<4, 2, HOOKS, false, 4, true>;
 
-// The prep kernel of the two-kernel path: the four producer waves alone (no
-// consumers, no V staging); they copy each chunk's tiles out themselves (kCopy).
-struct PrepVariant {
-  static constexpr bool kHooks = false, kCopy = true, kPipelined = false, kPersist = false;
-  static constexpr int NCW = 0, NP = 4, ROWS = 128, F = 1;
-  static constexpr int NTHREADS = 64 * (NCW + 4);
-  static constexpr int VSEG = 0;
-};
-
-// Prepared tiles of one chunk-head in the workspace, in 16-byte units: of the LDS
-// tiles of T~ hi, T~ lo and P, in that order, the part that the state pass reads
-// (the operand rows of the lower-triangular block pairs): rows 0 .. 31, columns
-// 0 .. 31 (4 units a row), then rows 32 .. 63, columns 0 .. 63 (8 units a row), in
-// the tiles' permuted column order, strictly-upper blocks zero; then the chunk's
-// gates beta_c, e^{gamma_c} and e^{gamma_last - gamma_c} (fp32, 64 each).  The
-// rest of each tile (columns 32 .. 63 of rows 0 .. 31, and the row padding) stays
-// zero in the state pass's LDS.  Chunk t of sequence s, v-head h is image (s TC +
-// t) Hv + h, TC = ceil(T / C) (a sequence clamped into [0, T] has at most TC chunks).
-constexpr int kTileUnits1 = 32 * 4 + 32 * 8;  // units of one tile
+// Prepared tiles of one chunk-head in the workspace (its image), in 16-byte units: the
+// operand fragments of T~ hi, T~ lo and P that the state pass reads, in that order, six
+// fragments each (tile_frag) of one unit per lane, so that an image is copied and its
+// fragments are read linearly; then the chunk's gates beta_c, e^{gamma_c} and
+// e^{gamma_last - gamma_c} (fp32, 64 each).  The strictly-upper blocks of fragments
+// (0, 0) and (2, 1) are zeros.  The chunks of a batch (of the window of it that a launch
+// covers) are numbered through, sequence after sequence (chunk_slots); chunk-head
+// (slot n, v-head h) is image n Hv + h.
+constexpr int kTileFrags = 6;
+constexpr int kTileUnits1 = kTileFrags * 64;  // units of one tile
 constexpr int kTileUnits = 3 * kTileUnits1;
 constexpr int kGateUnits = 3 * C / 4;
 constexpr int kTileImage = kTileUnits + kGateUnits;
 
-// Element offset, from the tile's base, of unit e (0 .. kTileUnits1 - 1) of a tile's
-// part of an image.
-__device__ __forceinline__ int tile_unit_off(int e) {
-  return e < 128 ? (e >> 2) * TSTR + 8 * (e & 3) : (32 + ((e - 128) >> 3)) * TSTR + 8 * ((e - 128) & 7);
-}
+// Fragment of a lower-triangular tile for rows 16 ct .. +15, contraction block js.
+__device__ __forceinline__ constexpr int tile_frag(int ct, int js) { return ct < 2 ? ct : 2 * ct - 2 + js; }
+
 constexpr int kMaxSortedSeqs = 1024;  // longest-first ordering up to this many sequences
 constexpr int kMaxPersistList = 128;  // chains per workgroup of the persistent kernel
 constexpr int kMaxPersistLpt = 64;    // batches of at most this many sequences get a longest-processing-time list
 
 struct __align__(16) PrefillSmem {
-  static constexpr int kParities = 2;  // chunk buffers in flight
   uint16_t K[2][C * KSTR];    // K chunk [c][perm(k)], by chunk parity
   uint16_t Q[2][C * KSTR];    // Q chunk [c][perm(k)]
   uint16_t Th[2][C * TSTR];   // T~ hi [c][perm(j)] (strictly-upper blocks stay 0)
@@ -216,39 +203,26 @@ static_assert(offsetof(PrefillSmem, Nh) % 16 == 0 &&
                   sizeof(PrefillSmem::Nh) + sizeof(PrefillSmem::Nl) >= kYxBytes,
               "Y exchange fits Nh and Nl");
 
-// LDS of the prep kernel (two-kernel path): one chunk's buffers (the producers
-// stage chunk t + 1 once the copier has written chunk t out) and no V, so that two
-// workgroups share a CU.
+// LDS of one wave of the prep kernel (two-kernel path), where a wave prepares a whole
+// chunk-head: what its lanes exchange.
 struct __align__(16) PrepSmem {
-  static constexpr int kParities = 1;
-  uint16_t K[1][C * KSTR];
-  uint16_t Q[1][C * KSTR];
-  uint16_t Th[1][C * TSTR];
-  uint16_t Tl[1][C * TSTR];
-  uint16_t P[1][C * TSTR];
-  uint16_t V[8];              // no V is staged (PrepVariant::VSEG = 0)
-  uint16_t Nh[NROWS * TSTR];
-  uint16_t Nl[NROWS * TSTR];
-  float Nd[4 * NDB];
-  float gam[1][C];
-  float gaml[1][C];
-  float bet[1][C];
-  float eg[1][C];
-  float dd[1][C];
-  int sync[16];
-  int spin_limit;
-  unsigned* aborts;
+  float gam[C];
+  float gaml[C];
+  float bet[C];
+  uint16_t D[2][4 * 16 * 16];  // diagonal blocks of T~, hi and lo, column-major ([block][col][row])
+  union {
+    float Nd[4 * NDB];              // diagonal blocks of N (until they are inverted)
+    uint16_t X[6][2][16 * 16];      // off-diagonal blocks of T~, hi and lo, column-major
+  };
 };
+static_assert(12 * sizeof(PrepSmem) <= 160 * 1024, "three prep waves a SIMD");
 
-// Gate arrays are copied to and from chunk images in 16-byte units, addressed from
-// beta (gate_unit): 16-byte aligned, e^gamma and the update decay following it.
-template <class Smem>
-constexpr bool gates_follow_beta() {
-  return offsetof(Smem, bet) % 16 == 0 && offsetof(Smem, eg) == offsetof(Smem, bet) + sizeof(Smem::bet) &&
-         offsetof(Smem, dd) == offsetof(Smem, eg) + sizeof(Smem::eg) &&
-         sizeof(Smem::bet) == Smem::kParities * C * sizeof(float);
-}
-static_assert(gates_follow_beta<PrefillSmem>() && gates_follow_beta<PrepSmem>(), "gate layout");
+// Gate arrays are copied from chunk images in 16-byte units, addressed from beta
+// (gate_unit): 16-byte aligned, e^gamma and the update decay following it.
+static_assert(offsetof(PrefillSmem, bet) % 16 == 0 &&
+                  offsetof(PrefillSmem, eg) == offsetof(PrefillSmem, bet) + sizeof(PrefillSmem::bet) &&
+                  offsetof(PrefillSmem, dd) == offsetof(PrefillSmem, eg) + sizeof(PrefillSmem::eg),
+              "gate layout");
 
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -313,6 +287,17 @@ __device__ __forceinline__ uint4 frag_kq(const uint16_t* tile, int row0, int ks,
 // stored with permuted columns.
 __device__ __forceinline__ uint4 frag(const uint16_t* tile, int stride, int row0, int ks, int lane) {
   return *reinterpret_cast<const uint4*>(tile + (row0 + (lane & 15)) * stride + 32 * ks + 8 * (lane >> 4));
+}
+
+// Operand row of a T~ or P tile, rows 16 ct + lane%16, contraction block js: from the
+// producers' row-major tile, or (state pass) from the copied image's fragments.
+template <bool kImage>
+__device__ __forceinline__ uint4 tile_row(const uint16_t* tile, int ct, int js, int lane) {
+  if constexpr (kImage) {
+    return *reinterpret_cast<const uint4*>(tile + 8 * (64 * tile_frag(ct, js) + lane));
+  } else {
+    return frag(tile, TSTR, 16 * ct, js, lane);
+  }
 }
 
 __device__ __forceinline__ uint2 read_tr(const uint16_t* p) {
@@ -405,9 +390,77 @@ __device__ __forceinline__ int64_t load_cu(const void* cu, int is64, int i) {
   return is64 ? static_cast<const int64_t*>(cu)[i] : int64_t(static_cast<const int32_t*>(cu)[i]);
 }
 
+// Tokens [s0, s1) of sequence i, its offsets clamped into [0, T].
+struct SeqRange {
+  int64_t s0, s1;
+};
+__device__ __forceinline__ SeqRange seq_range(const PrefillArgs& p, int i) {
+  int64_t a = load_cu(p.cu_seqlens, p.cu_is_64, i), b = load_cu(p.cu_seqlens, p.cu_is_64, i + 1);
+  a = a < 0 ? 0 : (a > p.T ? p.T : a);
+  b = b < a ? a : (b > p.T ? p.T : b);
+  return SeqRange{a, b};
+}
+
 template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_or_zero(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROW_MASK, 0xF, true));
+__device__ __forceinline__ int dpp_or_zero(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROW_MASK, 0xF, true);
+}
+
+// Inclusive prefix sum of an int over the wavefront (the DPP steps of
+// wave_inclusive_scan2).
+__device__ __forceinline__ int wave_inclusive_scan(int x) {
+  x += dpp_or_zero<0x111, 0xF>(x);
+  x += dpp_or_zero<0x112, 0xF>(x);
+  x += dpp_or_zero<0x114, 0xF>(x);
+  x += dpp_or_zero<0x118, 0xF>(x);
+  x += dpp_or_zero<0x142, 0xA>(x);
+  x += dpp_or_zero<0x143, 0xC>(x);
+  return x;
+}
+
+// Chunks of the sequences before sequence `seq` (a wave-uniform call of a whole wave):
+// the number of its first chunk among the batch's chunk images.  With valid offsets the
+// batch has at most T / C + N chunks, with any at most N ceil(T / C).
+__device__ int chunks_before(const PrefillArgs& p, int seq, int lane) {
+  int before = 0;
+  for (int base = 0; base < seq; base += 64) {
+    int n = 0;
+    if (base + lane < seq) {
+      const SeqRange r = seq_range(p, base + lane);
+      n = int((r.s1 - r.s0 + C - 1) / C);
+    }
+    before += __builtin_amdgcn_readlane(wave_inclusive_scan(n), 63);
+  }
+  return before;
+}
+
+// Chunk number `slot` of the batch: its first token and its length (0 if the batch has
+// fewer chunks), and the batch's number of chunks; wave-uniform.  (Token indices fit 31
+// bits.)
+struct ChunkAt {
+  int start, clen, total;
+};
+__device__ __forceinline__ ChunkAt find_chunk(const PrefillArgs& p, int slot, int lane) {
+  if (p.N == 1) {
+    const SeqRange r = seq_range(p, 0);
+    const int64_t cs = r.s0 + int64_t(slot) * C;
+    return ChunkAt{int(cs), cs >= r.s1 ? 0 : int(r.s1 - cs < C ? r.s1 - cs : C), int((r.s1 - r.s0 + C - 1) / C)};
+  }
+  ChunkAt c = {0, 0, 0};
+  for (int base = 0; base < p.N; base += 64) {
+    SeqRange r = {0, 0};
+    if (base + lane < p.N) r = seq_range(p, base + lane);
+    const int n = int((r.s1 - r.s0 + C - 1) / C);
+    const int end = wave_inclusive_scan(n) + c.total;
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(slot >= end - n && slot < end);
+    if (hit != 0) {
+      const int l = __builtin_ctzll(hit);
+      c.start = __builtin_amdgcn_readlane(int(r.s0), l) + C * (slot - __builtin_amdgcn_readlane(end - n, l));
+      c.clen = min(__builtin_amdgcn_readlane(int(r.s1), l) - c.start, C);
+    }
+    c.total = __builtin_amdgcn_readlane(end, 63);
+  }
+  return c;
 }
 
 template <int CTRL, int ROW_MASK>
@@ -539,8 +592,7 @@ __device__ __forceinline__ void signal_count(Smem& sm, int which, int lane) {
 // can cause), it raises kAbort, and all later waits return at once, so the
 // workgroup still finishes instead of hanging.  The wave that gives up adds 1 to
 // gdn_prefill_giveup_count (a global atomic from one lane), and the workgroup
-// writes NaN to every output element and state element it owns (and the prep
-// kernel NaN images), so wrong results never look valid.  Production kernels give
+// writes NaN to every output element and state element it owns, so wrong results never look valid.  Production kernels give
 // up after kSpinLimit polls; kernels built with the hooks after sm.spin_limit
 // polls, also counting each give-up in sm.aborts if set.
 template <bool kHooks, class Smem>
@@ -606,7 +658,6 @@ struct ChunkBufs {
 
 template <class Smem>
 __device__ __forceinline__ ChunkBufs chunk_bufs(Smem& sm, int b) {
-  b %= Smem::kParities;
   return ChunkBufs{sm.K[b],   sm.Q[b],   sm.Th[b],  sm.Tl[b], sm.P[b],
                    sm.gam[b], sm.gaml[b], sm.bet[b], sm.eg[b], sm.dd[b]};
 }
@@ -692,8 +743,8 @@ __device__ __forceinline__ void run_tiles(Smem& sm, const ChunkBufs& cb, const T
 
 // The four diagonal blocks of T~, D_I = (I + N_II)^-1.  diag_tiles forms N_II
 // from the tiles K_I K_I^T (scaled as in the off-diagonal epilogue) for blocks
-// I0 .. I1-1, stored column-major; diag_solve (one wavefront, all four blocks)
-// then has lane (r, j) = (lane/16, lane%16) invert block r, column j,
+// I0 .. I1-1, stored column-major; diag_solve (one wavefront, all four blocks;
+// diag_columns) then has lane (r, j) = (lane/16, lane%16) invert block r, column j,
 // x = D_r[:, j], by right-looking forward substitution:
 //   x_m = delta_mj - a_m,  a_i += N[i][m] x_m  for i > m
 // (for m < j every term is zero, so x_m = 0 there).  The column of N needed at
@@ -727,10 +778,9 @@ __device__ __forceinline__ void diag_tiles(Smem& sm, const ChunkBufs& cb, int la
   }
 }
 
-template <class Smem>
-__device__ __forceinline__ void diag_solve(Smem& sm, const ChunkBufs& cb, int lane) {
+__device__ __forceinline__ void diag_columns(const float* Nd, float (&x)[16], int lane) {
   const int r = lane >> 4, j = lane & 15;
-  const float* nb = sm.Nd + r * NDB;
+  const float* nb = Nd + r * NDB;
   // Columns are read kColAhead steps ahead of their use.
   constexpr int kColAhead = 4;
   f32x4 colv[15][4];
@@ -738,7 +788,7 @@ __device__ __forceinline__ void diag_solve(Smem& sm, const ChunkBufs& cb, int la
   for (int m = 0; m < kColAhead; ++m)
 #pragma unroll
     for (int q = (m + 1) / 4; q < 4; ++q) colv[m][q] = ld4(nb + m * 16 + 4 * q);
-  float a[16], x[16];
+  float a[16];
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
     x[m] = (m == j) ? 1.f : (m == 0 ? 0.f : -a[m]);
@@ -758,6 +808,13 @@ __device__ __forceinline__ void diag_solve(Smem& sm, const ChunkBufs& cb, int la
       }
     }
   }
+}
+
+template <class Smem>
+__device__ __forceinline__ void diag_solve(Smem& sm, const ChunkBufs& cb, int lane) {
+  const int r = lane >> 4, j = lane & 15;
+  float x[16];
+  diag_columns(sm.Nd, x, lane);
   // rows 16r + i, column 16r + j of T~
   const int colp = perm(16 * r + j);
 #pragma unroll
@@ -983,36 +1040,8 @@ __device__ __forceinline__ void stage_kq_gates(const ChunkBufs& cb, const Produc
 
 // Unit g of a chunk's gates (beta, e^gamma, e^{gamma_last - gamma}; 16 units each),
 // as an offset from beta, so that the address stays a known LDS address.
-template <class Smem>
 __device__ __forceinline__ float* gate_unit(const ChunkBufs& cb, int g) {
-  return cb.bet + (g >> 4) * (Smem::kParities * C) + 4 * (g & 15);
-}
-
-// Producer thread pt's share of a chunk's T~ hi, T~ lo and P tiles (the parts of
-// their LDS tiles that the state pass reads) and gates to the chunk's image in the
-// workspace; NaN images once a hand-off wait of the workgroup gave up.  The gates go
-// out from the first wave, which stores the next chunk's gates after this copy.
-template <class Smem>
-__device__ __forceinline__ void copy_tiles_out(const ChunkBufs& cb, u32x4* image, int pt, bool poison) {
-  constexpr int NT1 = kTileUnits1;
-  constexpr int NIT = (kTileUnits + NPROD - 1) / NPROD;
-  constexpr u32x4 nan4 = u32x4{kNaNx2, kNaNx2, kNaNx2, kNaNx2};
-  // All LDS reads first (one round of latency), then the stores; units past the
-  // tiles (last round) re-read the last unit and store nothing.
-  u32x4 v[NIT];
-#pragma unroll
-  for (int it = 0; it < NIT; ++it) {
-    const int e = pt + it * NPROD < kTileUnits ? pt + it * NPROD : kTileUnits - 1;
-    const uint16_t* src = e < NT1       ? cb.Th + tile_unit_off(e)
-                          : e < 2 * NT1 ? cb.Tl + tile_unit_off(e - NT1)
-                                        : cb.P + tile_unit_off(e - 2 * NT1);
-    v[it] = *reinterpret_cast<const u32x4*>(src);
-  }
-  const u32x4 gv = pt < kGateUnits ? *reinterpret_cast<const u32x4*>(gate_unit<Smem>(cb, pt)) : nan4;
-#pragma unroll
-  for (int it = 0; it < NIT; ++it)
-    if (pt + it * NPROD < kTileUnits) image[pt + it * NPROD] = poison ? nan4 : v[it];
-  if (pt < kGateUnits) image[kTileUnits + pt] = poison ? nan4 : gv;
+  return cb.bet + (g >> 4) * (2 * C) + 4 * (g & 15);
 }
 
 // Persistent kernel: the number of chains in the workgroup's list, and the first
@@ -1029,23 +1058,15 @@ __device__ __forceinline__ int next_chain(Smem& sm, int k) {
   return k;
 }
 
-// The producer loop: chunk t is prepared into the buffers of parity t & 1 (of
-// Smem::kParities) once the consumers are done with the chunk that used them last
-// (chunk t - 2 with two parities).  The four producer waves meet twice per chunk
+// The producer loop: chunk t is prepared into the buffers of parity t & 1 once the
+// consumers are done with the chunk that used them last (chunk t - 2).  The four producer waves meet twice per chunk
 // (after staging; after the tiles and diagonal blocks) on their own counter; the
 // chunk is handed over when all four are done.  V is staged for the workgroup's
 // state rows [row0, row0 + ROWS) only.
-// With V::kCopy (the prep kernel, no consumers) the producers also write each
-// chunk's tiles to images (chunk t of the run at images + t Hv kTileImage): chunk
-// t - 1's in step 1 of tick t, once all four waves have handed it over (so also
-// done with its K and Q, which the staging overwrites), and before the staging
-// barrier, after which tick t writes the same tiles; the first wave copies the
-// gates out before it stores the next chunk's.
 template <class V, class Smem>
 __device__ __forceinline__ void producer_loop(Smem& sm, const PrefillArgs& p, int64_t s0, int64_t s1,
-                                              int nchunks, int h, int hq, int hk, int row0, int pw, int lane0,
-                                              u32x4* images = nullptr) {
-  constexpr int NVIT = V::VSEG > 0 ? (V::VSEG + NPROD - 1) / NPROD : 1;  // V segments per producer thread
+                                              int nchunks, int h, int hq, int hk, int row0, int pw, int lane0) {
+  constexpr int NVIT = (V::VSEG + NPROD - 1) / NPROD;  // V segments per producer thread
   const int pt = pw * 64 + lane0;
   const float neg_decay = -expf(p.A_log[h]);
   const float dt_bias = p.dt_bias[h];
@@ -1108,21 +1129,11 @@ __device__ __forceinline__ void producer_loop(Smem& sm, const PrefillArgs& p, in
       }
     }
     const ChunkBufs cb = chunk_bufs(sm, u & 1);
-    // The buffers of chunk u - kParities (the same ones) consumed.
-    constexpr int kPar = Smem::kParities;
-    if (u >= kPar) wait_count<V::kHooks>(sm, kConsumed, V::NCW * (u - kPar + 1));
-    if constexpr (V::kCopy) {
-      if (t >= 1) wait_count<V::kHooks>(sm, kReady, 4 * t);  // chunk t - 1 handed over by all four waves
-    }
+    // The buffers of chunk u - 2 (the same ones) consumed.
+    if (u >= 2) wait_count<V::kHooks>(sm, kConsumed, V::NCW * (u - 1));
 
     // 1: stage K/Q (permuted columns), gates
     stage_kq(cb, f, pt);
-    if constexpr (V::kCopy) {
-      // Chunk t - 1's tiles out, after the staging: its stores are counted with the
-      // loads, and the staging's wait for its registers would wait for them too.
-      if (t >= 1)
-        copy_tiles_out<Smem>(chunk_bufs(sm, (t - 1) & 1), images + int64_t(t - 1) * p.Hv * kTileImage, pt, aborted(sm));
-    }
     if (pw == 0) store_gates(cb, gts, lane);
     // The V slice of this chunk into registers; staged at the end of the tick,
     // after the consumers' last read of the previous chunk's V.
@@ -1233,11 +1244,6 @@ __device__ __forceinline__ void producer_loop(Smem& sm, const PrefillArgs& p, in
     nchunks = int((s1 - s0 + C - 1) / C);
   }
   }
-  if constexpr (V::kCopy) {
-    wait_count<V::kHooks>(sm, kReady, 4 * nchunks);
-    copy_tiles_out<Smem>(chunk_bufs(sm, (nchunks - 1) & 1), images + int64_t(nchunks - 1) * p.Hv * kTileImage, pt,
-                   aborted(sm));
-  }
 }
 
 // The raw gate inputs (a, b) of token `lane` of a chunk, clamped into the chunk.
@@ -1275,7 +1281,7 @@ template <class V>
 __device__ __forceinline__ void producer_loop_split(PrefillSmem& sm, const PrefillArgs& p, int64_t s0, int64_t s1,
                                                     int nchunks, int h, int hq, int hk, int row0, int pw,
                                                     int lane0) {
-  static_assert(V::kPipelined && !V::kLoad && !V::kCopy, "pipelined producer loop of split chains");
+  static_assert(V::kPipelined && !V::kLoad, "pipelined producer loop of split chains");
   constexpr int NS = V::kStagers, NST = 64 * NS;        // stager waves, threads
   constexpr int NVIT = (V::VSEG + NST - 1) / NST;       // V segments per stager thread
   const int si = pw == 2 ? 0 : pw >= 4 ? pw - 3 : -1;   // stager index (waves 2, 4, 5, 6)
@@ -1526,12 +1532,12 @@ __device__ __forceinline__ void loader_loop(PrefillSmem& sm, const PrefillArgs& 
     for (int it = 0; it < NTIT; ++it) {
       const int e = pt + it * NPROD;
       if (e < kTileUnits) {
-        uint16_t* dst = e < NT1       ? cb.Th + tile_unit_off(e)
-                        : e < 2 * NT1 ? cb.Tl + tile_unit_off(e - NT1)
-                                      : cb.P + tile_unit_off(e - 2 * NT1);
+        uint16_t* dst = e < NT1       ? cb.Th + 8 * e
+                        : e < 2 * NT1 ? cb.Tl + 8 * (e - NT1)
+                                      : cb.P + 8 * (e - 2 * NT1);
         *reinterpret_cast<u32x4*>(dst) = tv[it];
       } else if (e < kTileImage) {
-        *reinterpret_cast<u32x4*>(gate_unit<PrefillSmem>(cb, e - kTileUnits)) = tv[it];
+        *reinterpret_cast<u32x4*>(gate_unit(cb, e - kTileUnits)) = tv[it];
       }
     }
     if (t >= 1) wait_count<V::kHooks>(sm, kVFree, V::NCW * t);  // the consumers' last read of V
@@ -1715,13 +1721,13 @@ __device__ __forceinline__ void consumer_loop(PrefillSmem& sm, const PrefillArgs
 #pragma unroll
         for (int js = 0; js <= (ct >> 1); ++js) {
           const int i = ct < 2 ? ct : 2 * ct - 2 + js;
-          thf[i] = frag(cb.Th, TSTR, 16 * ct, js, lane);
-          tlf[i] = frag(cb.Tl, TSTR, 16 * ct, js, lane);
+          thf[i] = tile_row<V::kLoad>(cb.Th, ct, js, lane);
+          tlf[i] = tile_row<V::kLoad>(cb.Tl, ct, js, lane);
         }
 #pragma unroll
       for (int js = 0; js < 2; ++js)
 #pragma unroll
-        for (int ct = 2 * js; ct < 4; ++ct) pqf[js ? ct + 2 : ct] = frag(cb.P, TSTR, 16 * ct, js, lane);
+        for (int ct = 2 * js; ct < 4; ++ct) pqf[js ? ct + 2 : ct] = tile_row<V::kLoad>(cb.P, ct, js, lane);
       __builtin_amdgcn_sched_barrier(0);
     }
     // v_new = T~ Y (contraction over the rows of Y in blocks js; T~ is lower triangular).
@@ -1742,8 +1748,8 @@ __device__ __forceinline__ void consumer_loop(PrefillSmem& sm, const PrefillArgs
           th = thf[ct < 2 ? ct : 2 * ct - 2 + js];
           tl = tlf[ct < 2 ? ct : 2 * ct - 2 + js];
         } else {
-          th = frag(cb.Th, TSTR, 16 * ct, js, lane);
-          tl = frag(cb.Tl, TSTR, 16 * ct, js, lane);
+          th = tile_row<V::kLoad>(cb.Th, ct, js, lane);
+          tl = tile_row<V::kLoad>(cb.Tl, ct, js, lane);
         }
 #pragma unroll
         for (int vt = 0; vt < VT; ++vt) {
@@ -1765,7 +1771,7 @@ __device__ __forceinline__ void consumer_loop(PrefillSmem& sm, const PrefillArgs
         if constexpr (VT == 1) {
           pq = pqf[js ? ct + 2 : ct];
         } else {
-          pq = frag(cb.P, TSTR, 16 * ct, js, lane);
+          pq = tile_row<V::kLoad>(cb.P, ct, js, lane);
         }
 #pragma unroll
         for (int vt = 0; vt < VT; ++vt) Xq[vt][ct] = mfma(vb[vt], pq, Xq[vt][ct]);
@@ -1912,12 +1918,12 @@ __device__ __forceinline__ void consumer_loop_tsplit(PrefillSmem& sm, const Pref
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int js = 0; js <= (c >> 1); ++js) {
-        const int i = c < 2 ? c : 2 * c - 2 + js;
-        thf[i] = frag(cb.Th, TSTR, 16 * c, js, lane);
-        tlf[i] = frag(cb.Tl, TSTR, 16 * c, js, lane);
+        const int i = tile_frag(c, js);
+        thf[i] = tile_row<true>(cb.Th, c, js, lane);
+        tlf[i] = tile_row<true>(cb.Tl, c, js, lane);
       }
-    const uint4 pq0 = frag(cb.P, TSTR, 16 * ct, 0, lane);
-    const uint4 pq1 = frag(cb.P, TSTR, 16 * ct, 1, lane);
+    const uint4 pq0 = tile_row<true>(cb.P, ct, 0, lane);
+    const uint4 pq1 = tile_row<true>(cb.P, ct, ct >> 1, lane);  // used by ct >= 2 only
     wait_count<V::kHooks>(sm, kYx, 4 * t);
     f32x4 Y[4];
 #pragma unroll
@@ -1933,7 +1939,7 @@ __device__ __forceinline__ void consumer_loop_tsplit(PrefillSmem& sm, const Pref
       Vn[c] = zero4();
 #pragma unroll
       for (int js = 0; js <= (c >> 1); ++js) {
-        const uint4 th = thf[c < 2 ? c : 2 * c - 2 + js], tl = tlf[c < 2 ? c : 2 * c - 2 + js];
+        const uint4 th = thf[tile_frag(c, js)], tl = tlf[tile_frag(c, js)];
         Vn[c] = mfma(th, Yh[js], Vn[c]);
         Vn[c] = mfma(th, Yl[js], Vn[c]);
         Vn[c] = mfma(tl, Yh[js], Vn[c]);
@@ -2090,8 +2096,8 @@ __global__ __launch_bounds__(V::NTHREADS) void gdn_prefill_kernel(PrefillArgs p)
   if (wave >= NCW) {
     if (nchunks > 0) {
       if constexpr (V::kLoad) {
-        const int64_t tc = (p.T + C - 1) / C;
-        const u32x4* tiles = reinterpret_cast<const u32x4*>(p.tiles) + (int64_t(seq) * tc * p.Hv + h) * kTileImage;
+        const u32x4* tiles = reinterpret_cast<const u32x4*>(p.tiles) +
+                             (int64_t(chunks_before(p, seq, lane0)) * p.Hv + h) * kTileImage;
         loader_loop<V>(sm, p, tiles, s0, s1, nchunks, h, hq, hk, row0, wave - NCW, lane0);
       } else {
         if constexpr (V::kPipelined) {
@@ -2414,58 +2420,235 @@ __global__ __launch_bounds__(V::NTHREADS) void gdn_prefill_persistent_kernel(Pre
   }
 }
 
-// Prep kernel of the two-kernel path (few chains).  Item (s R' + r) Hv + h (the
-// workgroup index paired as below) prepares chunks r p.prep_chunks .. (r + 1) p.prep_chunks - 1 of sequence s for
-// v-head h (R' = ceil(TC / p.prep_chunks)): the producer waves run their loop over
-// those chunks and copy each one's T~ hi, T~ lo and P tiles (LDS images) to its
-// image in p.tiles; their loads of chunk t + 1 are in flight meanwhile.  Its LDS
-// (PrepSmem, one chunk's buffers, no V) lets two workgroups share a CU.  Chunks are
-// independent, so all of them are prepared at once; the state pass (Variant<..,
-// LOAD = true>) then only copies them.
-__global__ __launch_bounds__(PrepVariant::NTHREADS) void gdn_prefill_prep_kernel(PrefillArgs p) {
-  constexpr int NTHREADS = PrepVariant::NTHREADS;
-  __shared__ PrepSmem sm;
-  const int tid = threadIdx.x;
-  const int lane0 = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t tc = (p.T + C - 1) / C;
-  const int run = p.prep_chunks;
-  const int64_t runs = (tc + run - 1) / run;
-  // Workgroups are dealt to the 8 XCDs round-robin: blocks b and b + 8 of each group
-  // of 16 take items 2m and 2m + 1 (v-heads 2j and 2j + 1 of one run, which read the
-  // same K and Q), so the two share an XCD's L2.
-  const int64_t b = blockIdx.x;
-  const int64_t bid = (b & ~int64_t(15)) | ((b & 7) << 1) | ((b >> 3) & 1);
-  if (bid >= int64_t(p.N) * runs * p.Hv) return;  // padding of the last group of 16 (workgroup-uniform)
-  const int h = int(bid % p.Hv);
-  const int seq = int(bid / p.Hv / runs), r = int(bid / p.Hv % runs);
-  int64_t s0 = load_cu(p.cu_seqlens, p.cu_is_64, seq);
-  int64_t s1 = load_cu(p.cu_seqlens, p.cu_is_64, seq + 1);
-  s0 = s0 < 0 ? 0 : (s0 > p.T ? p.T : s0);
-  s1 = s1 < s0 ? s0 : (s1 > p.T ? p.T : s1);
-  const int64_t t0 = int64_t(r) * run;           // first chunk of the run
-  const int64_t cs = s0 + t0 * C;
-  if (cs >= s1) return;  // the sequence has no chunk t0 (workgroup-uniform)
-  const int64_t ce = s1 - cs < int64_t(run) * C ? s1 : cs + int64_t(run) * C;
-  const int nchunks = int((ce - cs + C - 1) / C);
+// ---------------------------------------------------------------------------
+// Prep kernel of the two-kernel path: T~, P and the gates of every chunk-head, one
+// wave each.
+// ---------------------------------------------------------------------------
+
+// Rows 16 I + lane%16 of a chunk's K or Q slice (stride: bytes from token to token) as
+// operands in kappa order, contraction blocks ks = 0 .. 3.  A lane loads 16 contiguous
+// bytes a block (columns 32 ks + 8g .. +7, pieces 2g and 2g + 1 of four columns; rows past
+// the chunk lie outside the buffer and read as zeros), and two row swaps deal the eight
+// pieces of a row to its four lanes as kappa has them (lane g: pieces g and g + 4).  The
+// order is that of the producers' LDS tiles, so the products are the same bit for bit.
+struct RowFrags {
+  u32x4 v[4];
+  __device__ __forceinline__ void load(BufferRsrc r, int stride, int I, int lane) {
+    const int off = (16 * I + (lane & 15)) * stride + 16 * (lane >> 4);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) v[ks] = __builtin_amdgcn_raw_buffer_load_b128(r, off + 64 * ks, 0, 0);
+  }
+  __device__ __forceinline__ void to_kappa() {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const auto x = __builtin_amdgcn_permlane16_swap(v[ks][i], v[ks][2 + i], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
+        v[ks][i] = y[0];
+        v[ks][2 + i] = y[1];
+      }
+  }
+};
+
+__device__ __forceinline__ f32x4 row_product(const RowFrags& a, const RowFrags& b) {
+  f32x4 acc = zero4();
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+    acc = mfma(__builtin_bit_cast(uint4, a.v[ks]), __builtin_bit_cast(uint4, b.v[ks]), acc);
+  return acc;
+}
+
+// Four rows 4g .. +3 of column lane%16 of a 16x16 block stored column-major (a 16x16x16 B
+// operand), and row lane%16, columns 4g .. +3 (an A operand), by a transpose read.
+__device__ __forceinline__ uint2 block_rows_of_col(const uint16_t* blk, int lane) {
+  return *reinterpret_cast<const uint2*>(blk + 16 * (lane & 15) + 4 * (lane >> 4));
+}
+__device__ __forceinline__ uint2 block_cols_of_row(const uint16_t* blk, int lane) {
+  return read_tr(blk + 16 * (4 * (lane >> 4) + ((lane & 15) >> 2)) + 4 * (lane & 3));
+}
+
+// A block X (accumulator layout), split, as an A operand, through the wave's LDS.
+__device__ __forceinline__ void put_block(uint16_t (&blk)[2][256], const f32x4& X, int lane) {
+  uint2 hi, lo;
+  split4(X, hi, lo);
+  *reinterpret_cast<uint2*>(blk[0] + 16 * (lane & 15) + 4 * (lane >> 4)) = hi;
+  *reinterpret_cast<uint2*>(blk[1] + 16 * (lane & 15) + 4 * (lane >> 4)) = lo;
+}
+__device__ __forceinline__ Pair2 get_block(const uint16_t (&blk)[2][256], int lane) {
+  return Pair2{block_cols_of_row(blk[0], lane), block_cols_of_row(blk[1], lane)};
+}
+
+// Wave item (chunk number, v-head) prepares that chunk-head: the same values, from the same
+// operations in the same order, as the producers of the one-kernel path, but without their
+// hand-offs.  K and Q rows go from global memory into the operands, the N tiles stay in
+// registers (an N tile's accumulator layout is the A operand the off-diagonal solve takes),
+// the tiles (I, J) of N and P share their decays, and every fragment of the image leaves
+// the registers as a linear 16-byte store.  A chunk-head is a chain of dependent steps
+// (about 9k cycles of arithmetic and 5k of first loads), so what counts is how many are in
+// flight: 12 waves a CU, no barriers.  One 4,096-token sequence at 32 v-heads (2,048
+// chunk-heads, 72 MB of K, Q and images, inputs from HBM) takes 20.6 us, 12,288 tokens
+// 51.7; a workgroup of four waves per run of chunks, handing over through the LDS (two
+// workgroups a CU), took 26.9 and about 80.
+constexpr int kPrepWaves = 2;
+__global__ __launch_bounds__(64 * kPrepWaves, 2) void gdn_prefill_prep_kernel(PrefillArgs p) {
+  __shared__ PrepSmem smem[kPrepWaves];
+  const int lane0 = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  PrepSmem& sm = smem[wave];
+  // v-heads 2j and 2j + 1 of a chunk, which read the same K and Q, share a workgroup.
+  const int item = int(blockIdx.x) * kPrepWaves + wave;
+  const int h = item % p.Hv;
   const int hq = h / (p.Hv / p.Hq);
   const int hk = h / (p.Hv / p.Hk);
-
-  // Blocks never written per chunk are zeros (as in the one-kernel path).
-  const uint4 z = uint4{0u, 0u, 0u, 0u};
-  for (int e = tid; e < C * TSTR / 8; e += NTHREADS) {
-    reinterpret_cast<uint4*>(sm.P[0])[e] = z;
-    reinterpret_cast<uint4*>(sm.Th[0])[e] = z;
-    reinterpret_cast<uint4*>(sm.Tl[0])[e] = z;
-    if (e < NROWS * TSTR / 8) {
-      reinterpret_cast<uint4*>(sm.Nh)[e] = z;
-      reinterpret_cast<uint4*>(sm.Nl)[e] = z;
+  const float neg_decay = -expf(p.A_log[h]), dt_bias = p.dt_bias[h];
+  // One pass, except for malformed offsets whose sequences overlap: their chunks can
+  // exceed prep_slots.  (Items past the last chunk-head have slot >= prep_slots.)
+  for (int slot = item / p.Hv;; slot += p.prep_slots) {
+    int lane = lane0;  // opaque, so that lane-dependent addresses are not hoisted and spilled
+    asm volatile("" : "+v"(lane));
+    const int g = lane >> 4, n16 = lane & 15;
+    const ChunkAt c = find_chunk(p, slot, lane);
+    if (c.clen <= 0) break;
+    const int64_t cs = c.start;
+    const int clen = c.clen;
+    u32x4* image = reinterpret_cast<u32x4*>(p.tiles) + (int64_t(slot) * p.Hv + h) * kTileImage;
+    const int kstr = p.Hk * D * 2, qstr = p.Hq * D * 2;
+    const BufferRsrc kr = buffer_rsrc(const_cast<uint16_t*>(p.k) + (cs * p.Hk + hk) * D, uint32_t(clen - 1) * kstr + 2 * D);
+    const BufferRsrc qr = buffer_rsrc(const_cast<uint16_t*>(p.q) + (cs * p.Hq + hq) * D, uint32_t(clen - 1) * qstr + 2 * D);
+    ProducerPrefetch f;
+    {
+      const int row = lane < clen ? lane : clen - 1;
+      f.a = (p.a + cs * p.Hv + h)[row * p.Hv];
+      f.b = (p.b + cs * p.Hv + h)[row * p.Hv];
     }
+    // The loads go out two row blocks ahead of their use: a wave that issued all of them
+    // at once would wait for the memory queue, and all waves for the same memory, before
+    // any of them computes.
+    RowFrags k[4], q[4];
+    auto load_block = [&](int I) {
+      k[I].load(kr, kstr, I, lane);
+      q[I].load(qr, qstr, I, lane);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load_block(0);
+    load_block(1);
+    {
+      const ChunkGates gts = chunk_gates(f, lane, clen, neg_decay, dt_bias);
+      sm.gam[lane] = gts.gam;
+      sm.gaml[lane] = gts.gaml;
+      sm.bet[lane] = gts.bet;
+      float* gi = reinterpret_cast<float*>(image + kTileUnits);
+      gi[lane] = gts.bet;
+      gi[C + lane] = gts.eg;
+      gi[2 * C + lane] = gts.dd;
+    }
+    wave_lds_sync();
+
+    // Tiles (I, J), J <= I: decay e^{gamma_r - gamma_c} for r = 16I + n16, c = 16J + 4g + i;
+    // N[r][c] from k_c . k_r (off-diagonal: an A operand; diagonal: fp32, column-major) and
+    // P[r][c] from k_c . q_r (c <= r), with the output scale folded in.
+    Pair2 n[4][3];
+#pragma unroll
+    for (int I = 0; I < 4; ++I) {
+      if (I < 2) load_block(I + 2);
+      k[I].to_kappa();
+      q[I].to_kappa();
+      const int r = 16 * I + n16;
+      const float gr = sm.gam[r], grl = sm.gaml[r], br = sm.bet[r];
+      uint2 pt[4] = {uint2{0u, 0u}, uint2{0u, 0u}, uint2{0u, 0u}, uint2{0u, 0u}};
+#pragma unroll
+      for (int J = 0; J <= I; ++J) {
+        const f32x4 an = row_product(k[J], k[I]), ap = row_product(k[J], q[I]);
+        const f32x4 gcv = ld4(sm.gam + 16 * J + 4 * g), gcl = ld4(sm.gaml + 16 * J + 4 * g);
+        f32x4 e, x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          e[i] = exp2_le0(fminf(gamma_diff(gr, grl, gcv[i], gcl[i]), 0.f));
+          x[i] = br * e[i] * an[i];
+        }
+        if (J < I) {
+          split4(x, n[I][J < 3 ? J : 0].h, n[I][J < 3 ? J : 0].l);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sm.Nd[I * NDB + (4 * g + i) * 16 + n16] = x[i];
+        }
+        float pv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float y = e[i] * (ap[i] * p.scale);
+          pv[i] = J < I || 4 * g + i <= n16 ? y : 0.f;
+        }
+        pt[J] = uint2{pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3])};
+      }
+#pragma unroll
+      for (int js = 0; js <= I / 2; ++js)
+        image[2 * kTileUnits1 + 64 * tile_frag(I, js) + lane] =
+            u32x4{pt[2 * js].x, pt[2 * js].y, pt[2 * js + 1].x, pt[2 * js + 1].y};
+    }
+    wave_lds_sync();
+
+    // Diagonal blocks of T~: lane (r, j) forms column j of block r.
+    {
+      float x[16];
+      diag_columns(sm.Nd, x, lane);
+      uint2 hi[4], lo[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) split4(f32x4{x[4 * m], x[4 * m + 1], x[4 * m + 2], x[4 * m + 3]}, hi[m], lo[m]);
+      uint4* dh = reinterpret_cast<uint4*>(sm.D[0] + 16 * lane);
+      uint4* dl = reinterpret_cast<uint4*>(sm.D[1] + 16 * lane);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        dh[m] = uint4{hi[2 * m].x, hi[2 * m].y, hi[2 * m + 1].x, hi[2 * m + 1].y};
+        dl[m] = uint4{lo[2 * m].x, lo[2 * m].y, lo[2 * m + 1].x, lo[2 * m + 1].y};
+      }
+    }
+    wave_lds_sync();
+
+    // Off-diagonal blocks (the products and order of offdiag_right and offdiag_left).
+    Pair2 a[4], d[3];  // D_I as A operands, D_0 .. D_2 as B operands
+#pragma unroll
+    for (int I = 0; I < 4; ++I) {
+      a[I] = Pair2{block_cols_of_row(sm.D[0] + 256 * I, lane), block_cols_of_row(sm.D[1] + 256 * I, lane)};
+      if (I < 3) d[I] = Pair2{block_rows_of_col(sm.D[0] + 256 * I, lane), block_rows_of_col(sm.D[1] + 256 * I, lane)};
+    }
+    const f32x4 g32 = mul3_16(zero4(), n[3][2], d[2]);
+    const f32x4 g10 = mul3_16(zero4(), n[1][0], d[0]);
+    const f32x4 m21 = mul3_16(zero4(), n[2][1], d[1]);
+    const f32x4 m31 = mul3_16(zero4(), n[3][1], d[1]);
+    const f32x4 p20 = mul3_16(zero4(), n[2][0], d[0]);
+    const f32x4 p30 = mul3_16(zero4(), n[3][0], d[0]);
+    const Pair2 ng32 = acc_b(-g32), ng10 = acc_b(-g10), nm21 = acc_b(-m21), nm31 = acc_b(-m31);
+    put_block(sm.X[5], mul3_16(zero4(), a[3], ng32), lane);  // X32
+    const f32x4 x10 = mul3_16(zero4(), a[1], ng10);
+    const Pair2 x32t = acc_b(mul3_16(zero4(), ng32, a[3]));
+    put_block(sm.X[0], x10, lane);  // X10
+    const Pair2 b10 = acc_b(x10);
+    const Pair2 nm20 = acc_b(-mul3_16(p20, n[2][1], b10));
+    const Pair2 nm30 = acc_b(-mul3_16(p30, n[3][1], b10));
+    put_block(sm.X[2], mul3_16(zero4(), a[2], nm21), lane);                                  // X21
+    put_block(sm.X[4], mul3_16(mul3_16(zero4(), x32t, nm21), a[3], nm31), lane);             // X31
+    put_block(sm.X[1], mul3_16(zero4(), a[2], nm20), lane);                                  // X20
+    wave_lds_sync();
+    const Pair2 x32 = get_block(sm.X[5], lane);
+    put_block(sm.X[3], mul3_16(mul3_16(zero4(), a[3], nm30), x32, nm20), lane);              // X30
+    wave_lds_sync();
+    const Pair2 t10 = get_block(sm.X[0], lane), t20 = get_block(sm.X[1], lane), t21 = get_block(sm.X[2], lane),
+                t30 = get_block(sm.X[3], lane), t31 = get_block(sm.X[4], lane);
+    const Pair2 zero = {uint2{0u, 0u}, uint2{0u, 0u}};
+    auto store_frag = [&](int frag, const Pair2& left, const Pair2& right) {
+      image[64 * frag + lane] = u32x4{left.h.x, left.h.y, right.h.x, right.h.y};
+      image[kTileUnits1 + 64 * frag + lane] = u32x4{left.l.x, left.l.y, right.l.x, right.l.y};
+    };
+    store_frag(tile_frag(0, 0), a[0], zero);
+    store_frag(tile_frag(1, 0), t10, a[1]);
+    store_frag(tile_frag(2, 0), t20, t21);
+    store_frag(tile_frag(2, 1), a[2], zero);
+    store_frag(tile_frag(3, 0), t30, t31);
+    store_frag(tile_frag(3, 1), x32, a[3]);
+    if (slot + p.prep_slots >= c.total) break;
+    wave_lds_sync();
   }
-  if (tid < 16) sm.sync[tid] = 0;
-  __syncthreads();
-  u32x4* images = reinterpret_cast<u32x4*>(p.tiles) + ((int64_t(seq) * tc + t0) * p.Hv + h) * kTileImage;
-  producer_loop<PrepVariant>(sm, p, cs, ce, nchunks, h, hq, hk, 0, wave, lane0, images);
 }
 
 // `done`, if not null, is recorded by the launch itself when the kernel completes
@@ -2736,16 +2919,12 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream, hipEvent_t d
     }
   }
   if (a.tiles != nullptr && prefill_workspace_bytes(a.N, a.T, a.Hv) > 0) {
-    // Runs of consecutive chunks per prep workgroup, about two workgroups per CU
-    // for the batch's chunks (at most T / C + N of them).
+    // One prep wave per chunk-head; valid offsets give at most T / C + N chunks.
     const int64_t tc = (a.T + C - 1) / C;
-    const int64_t chunks = a.T / C + a.N < a.N * tc ? a.T / C + a.N : a.N * tc;
-    const int64_t slots = 2 * int64_t(device_cus());
-    const int64_t run = (chunks * a.Hv + slots - 1) / slots;
     PrefillArgs b = a;
-    b.prep_chunks = int(run < 1 ? 1 : run > tc ? tc : run);
-    const int64_t grid = (int64_t(a.N) * ((tc + b.prep_chunks - 1) / b.prep_chunks) * a.Hv + 15) / 16 * 16;
-    hipLaunchKernelGGL(gdn_prefill_prep_kernel, dim3(unsigned(grid)), dim3(PrepVariant::NTHREADS), 0, stream, b);
+    b.prep_slots = int(tc + a.N - 1 < a.N * tc ? tc + a.N - 1 : a.N * tc);
+    const int64_t grid = (int64_t(b.prep_slots) * a.Hv + kPrepWaves - 1) / kPrepWaves;
+    hipLaunchKernelGGL(gdn_prefill_prep_kernel, dim3(unsigned(grid)), dim3(64 * kPrepWaves), 0, stream, b);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (F == 4) return launch_variant<Variant<2, 1, false, true>>(a, stream, done);

@@ -418,6 +418,42 @@ def test_prefill_dropin_random_long_batches(gpu, seed):
     assert binding.prefill_giveups() == 0
 
 
+@pytest.mark.parametrize("lens,heads", [
+    ([int(x) for x in np.random.default_rng(91).integers(0, 131, 64)], Heads(1, 1, 1)),  # 64 sequences, one head
+    ([65, 0, 1, 64, 127], Heads(3, 1, 3)),          # odd heads: a prep workgroup spans two chunks
+    ([129, 700], Heads(2, 8, 16)),                  # distinct q and k ratios
+])
+def test_prefill_prep_kernel_edges(gpu, lens, heads):
+    """The prep kernel (a wave per chunk-head) where its indexing can go wrong: many
+    sequences, odd head counts, ragged and empty sequences.  Bit for bit gdn_prefill's
+    one kernel, and within tolerance of the oracle."""
+    say(f"prefill prep kernel edges lens={lens} heads={heads}")
+    p = workloads.prefill_inputs(lens, heads, seed=92, gate="slow", state_scale=0.5)
+    o1, s1 = _prefill_capi(p, gpu, workspace=False)
+    o2, s2 = _prefill_capi(p, gpu, workspace=True)
+    assert torch.equal(o1, o2) and torch.equal(s1, s2)
+    o_ref, s_ref = oracle_prefill(p)
+    assert_close(host(o2), o_ref, OUT_RTOL, OUT_ATOL, "output")
+    assert_close(host(s2), s_ref, STATE_RTOL, STATE_ATOL, "new_state")
+
+
+def test_prefill_two_kernels_overlapping_offsets(gpu):
+    """Malformed offsets on the two-kernel path: cu = [0, 200, 0, 200, 90] with T = 200
+    gives [0, 200), an empty sequence, [0, 200) again and an empty one: eight chunks, more
+    than any valid offsets of four sequences give (seven).  Both final states are those of
+    the 200 tokens; the outputs belong to two sequences and are not compared."""
+    say("prefill two kernels, overlapping offsets")
+    heads = Heads(2, 2, 4)
+    p = workloads.prefill_inputs([200], heads, seed=93, gate="slow", state_scale=0.5)
+    state = 0.5 * torch.randn((4, 4, 128, 128), generator=torch.Generator().manual_seed(93))
+    bad = dict(p, state=state, cu_seqlens=torch.tensor([0, 200, 0, 200, 90], dtype=torch.int32))
+    _, ns = _prefill_capi(bad, gpu, workspace=True)
+    for i in (0, 2):
+        _, s_ref = oracle_prefill(dict(p, state=state[i:i + 1], cu_seqlens=torch.tensor([0, 200], dtype=torch.int32)))
+        assert_close(host(ns[i]), s_ref[0], STATE_RTOL, STATE_ATOL, f"seq {i} state")
+    assert torch.equal(ns[1].cpu(), state[1]) and torch.equal(ns[3].cpu(), state[3])
+
+
 def test_prefill_workspace_reuse(gpu):
     """One workspace buffer, not cleared between calls, serves two different few-chain
     batches in turn (the larger first, then a smaller one whose images overlay the
