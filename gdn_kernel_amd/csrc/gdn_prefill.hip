@@ -88,8 +88,7 @@ constexpr int TSTR = 72;     // bf16 row stride of 64-wide tiles (T~, P, N)
 constexpr int NDB = 16 * 16 + 4;  // floats per diagonal N block (column-major; padded by 16 bytes)
 constexpr int NROWS = C - 16;  // rows of N kept for the off-diagonal solve
 
-template <int NCW_, int VT_, bool HOOKS_ = false, bool LOAD_ = false, int NP_ = 4, bool PERSIST_ = false,
-          bool TSPLIT_ = false, bool DEEP_ = false>
+template <int NCW_, int VT_, bool HOOKS_ = false, bool LOAD_ = false, int NP_ = 4, bool PERSIST_ = false>
 struct Variant {
   static constexpr bool kHooks = HOOKS_;         // testing hooks of PrefillArgs compiled in
   static constexpr bool kLoad = LOAD_;           // waves NCW.. load prepared T~/P (two-kernel path)
@@ -97,10 +96,7 @@ struct Variant {
   static constexpr int NP = NP_;                 // producer (or loader) waves: 4; or 7 (6) beside one (two) consumers
   static constexpr int VT = VT_;                 // 16-row state tiles per consumer wave
   static constexpr int VW = 16 * VT;             // state rows per consumer wave
-  // Token-split state pass (consumer_loop_tsplit): the consumer waves hold the same
-  // 16 state rows and share each chunk's tokens.
-  static constexpr bool kTokenSplit = TSPLIT_;
-  static constexpr int ROWS = TSPLIT_ ? VW : NCW * VW;  // state rows per workgroup
+  static constexpr int ROWS = NCW * VW;          // state rows per workgroup
   static constexpr int F = 128 / ROWS;           // workgroups per chain
   static constexpr int NTHREADS = 64 * (NCW + NP);
   static constexpr int VSEG = 8 * ROWS;          // 16-byte segments of the V slice of a chunk
@@ -115,11 +111,6 @@ struct Variant {
   // (gdn_prefill_persistent_kernel); the four-producer F = 1 layout only.
   static constexpr bool kPersist = PERSIST_;
   static_assert(!PERSIST_ || (NCW_ == 4 && VT_ == 2 && NP_ == 4 && !LOAD_), "persistent: F = 1 only");
-  static_assert(!TSPLIT_ || (NCW_ == 4 && VT_ == 1 && NP_ == 4 && LOAD_ && !PERSIST_), "token split: state pass, F = 8");
-  // State pass over images that the caches do not hold (long batches): the loaders
-  // load each chunk's images two chunks ahead instead of one.
-  static constexpr bool kDeepImages = DEEP_;
-  static_assert(!DEEP_ || LOAD_, "image prefetch depth: state pass only");
 };
 
 // Production launch variants by split factor F (workgroups per chain).  With F = 8
@@ -193,15 +184,6 @@ struct __align__(16) PrefillSmem {
 // kMaxSortedSeqs sequences in V.
 static_assert(kMaxSortedSeqs * sizeof(int) <= sizeof(PrefillSmem::Nh), "sequence lengths fit Nh");
 static_assert(3 * kMaxSortedSeqs * sizeof(int) <= sizeof(PrefillSmem::V), "sequence lists fit V");
-
-// The token-split state pass exchanges Y and the state's bf16 hi/lo parts through
-// Nh/Nl (unused without producers): four 16-token blocks of Y and four 32-column
-// blocks of the state, 16 and 32 bytes per lane.
-constexpr int kYxBytes = 4 * 64 * 16 + 4 * 64 * 32;
-static_assert(offsetof(PrefillSmem, Nh) % 16 == 0 &&
-                  offsetof(PrefillSmem, Nl) == offsetof(PrefillSmem, Nh) + sizeof(PrefillSmem::Nh) &&
-                  sizeof(PrefillSmem::Nh) + sizeof(PrefillSmem::Nl) >= kYxBytes,
-              "Y exchange fits Nh and Nl");
 
 // LDS of one wave of the prep kernel (two-kernel path), where a wave prepares a whole
 // chunk-head: what its lanes exchange.
@@ -551,9 +533,7 @@ enum SyncCounter {
   kStaged = 7,    // pipelined: the chunk's K/Q staged and its gates stored (NS + 1 a chunk)
   kNRead = 8,     // pipelined: the left off-diagonal wave read its N operands
   kVStaged = 9,   // pipelined: the chunk's V staged (NS a chunk)
-  kList = 10,     // persistent kernel: the workgroup's chain list is complete (1)
-  kYx = 11,       // token-split state pass: a consumer wave stored its block of Y (4 a chunk)
-  kSx = 12        // token-split state pass: a consumer wave stored its state columns (4 a chunk, 4 at start)
+  kList = 10      // persistent kernel: the workgroup's chain list is complete (1)
 };
 constexpr int kSpinLimit = 1 << 21;  // default polls (about 70 ms) before a wait gives up
 
@@ -602,7 +582,9 @@ __device__ __forceinline__ void wait_count(Smem& sm, int which, int target) {
       __builtin_amdgcn_s_sleep(1);
       if (__hip_atomic_load(&sm.sync[which], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= target) break;
       if (__hip_atomic_load(&sm.sync[kAbort], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0) break;
-      if (it >= (kHooks ? sm.spin_limit : kSpinLimit)) {
+      int limit = kSpinLimit;
+      if constexpr (kHooks) limit = sm.spin_limit;
+      if (it >= limit) {
         __hip_atomic_store(&sm.sync[kAbort], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) == 0) {
           __hip_atomic_fetch_add(&gdn_prefill_giveup_count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1461,8 +1443,7 @@ __device__ __forceinline__ void producer_loop_split(PrefillSmem& sm, const Prefi
 // computed.  K and Q are staged as the producers stage them, V at the end of the
 // tick, after the consumers' last read of the previous chunk's V.
 // The images of chunk t + 1 are loaded into registers during tick t, so their
-// latency overlaps the waits for the consumers; with V::kDeepImages the images of
-// chunk t + 2 (two register sets, alternating), as soon as chunk t's are in LDS.
+// latency overlaps the waits for the consumers.
 // V goes two chunks ahead in every variant (two register sets): the prep kernel does
 // not read V, so with inputs that the caches do not hold its loads come from HBM
 // (config 3 with four rotating input sets: 142.5 -> 132.0 us, unchanged with one).
@@ -1488,8 +1469,7 @@ __device__ __forceinline__ void loader_loop(PrefillSmem& sm, const PrefillArgs& 
 #pragma unroll
   for (int it = 0; it < NTIT; ++it) toff[it] = pt + it * NPROD < kTileImage ? pt + it * NPROD : kTileImage - 1;
   // (First-class vectors: copies of uint4 structs would go through the stack.)
-  constexpr bool deep = V::kDeepImages;
-  u32x4 tva[NTIT], tvb[deep ? NTIT : 1], fva[NVIT], fvb[NVIT];
+  u32x4 tv[NTIT], fva[NVIT], fvb[NVIT];
   // V slice of chunk t (tokens [s0 + C t, s1) of it) into fv, zero past the sequence.
   auto load_v = [&](int t, u32x4(&fv)[NVIT]) {
     const int64_t vs = s0 + int64_t(t) * C;
@@ -1503,23 +1483,16 @@ __device__ __forceinline__ void loader_loop(PrefillSmem& sm, const PrefillArgs& 
   };
   ProducerPrefetch f;
   producer_prefetch(p, s0, int(s1 - s0 < C ? s1 - s0 : C), h, hq, hk, pt, lo, f);
-  // Chunk 0's images (and chunk 1's), and the V slices of chunks 0 and 1, into registers.
+  // Chunk 0's images, and the V slices of chunks 0 and 1, into registers.
 #pragma unroll
-  for (int it = 0; it < NTIT; ++it) tva[it] = tiles[toff[it]];
-  if constexpr (deep) {
-    if (nchunks > 1) {
-      const u32x4* src = tiles + int64_t(p.Hv) * kTileImage;
-#pragma unroll
-      for (int it = 0; it < NTIT; ++it) tvb[it] = src[toff[it]];
-    }
-  }
+  for (int it = 0; it < NTIT; ++it) tv[it] = tiles[toff[it]];
   load_v(0, fva);
   if (nchunks > 1) load_v(1, fvb);
 
-  // Tick t stages chunk t from the register sets tv (images) and fv (V), then loads
+  // Tick t stages chunk t from the registers tv (images) and fv (V), then loads
   // chunk t + 2's V into fv (the V loads go two chunks ahead, so that their latency
   // from HBM, when the inputs are not in the caches, stays off the chain).
-  auto tick = [&](int t, u32x4(&tv)[NTIT], u32x4(&fv)[NVIT]) {
+  auto tick = [&](int t, u32x4(&fv)[NVIT]) {
     int lane = lane0;
     asm volatile("" : "+v"(lane));
     const int64_t cs = s0 + int64_t(t) * C;
@@ -1553,12 +1526,7 @@ __device__ __forceinline__ void loader_loop(PrefillSmem& sm, const PrefillArgs& 
     // them: the K/Q loads are conditional, so the compiler cannot count them and
     // waits for every load issued since.
     if (ncs < s1) producer_prefetch(p, ncs, nclen, h, hq, hk, pt, lo, f);
-    if (deep && t + 2 < nchunks) {  // chunk t + 2's images into this set
-      const u32x4* src = tiles + int64_t(t + 2) * p.Hv * kTileImage;
-#pragma unroll
-      for (int it = 0; it < NTIT; ++it) tv[it] = src[toff[it]];
-    }
-    if (!deep && t + 1 < nchunks) {  // chunk t + 1's images into registers
+    if (t + 1 < nchunks) {  // chunk t + 1's images into registers
       const u32x4* src = tiles + int64_t(t + 1) * p.Hv * kTileImage;
 #pragma unroll
       for (int it = 0; it < NTIT; ++it) tv[it] = src[toff[it]];
@@ -1566,14 +1534,8 @@ __device__ __forceinline__ void loader_loop(PrefillSmem& sm, const PrefillArgs& 
     if (t + 2 < nchunks) load_v(t + 2, fv);  // chunk t + 2's V slice
   };
   for (int t = 0; t < nchunks; t += 2) {
-    tick(t, tva, fva);
-    if (t + 1 < nchunks) {
-      if constexpr (deep) {
-        tick(t + 1, tvb, fvb);
-      } else {
-        tick(t + 1, tva, fvb);
-      }
-    }
+    tick(t, fva);
+    if (t + 1 < nchunks) tick(t + 1, fvb);
   }
 }
 
@@ -1829,173 +1791,12 @@ __device__ __forceinline__ void consumer_loop(PrefillSmem& sm, const PrefillArgs
   }
 }
 
-// The token-split consumer loop of the two-kernel state pass (F = 8).  The four
-// consumer waves share the slice's 16 state rows: wave w keeps state columns
-// 32w .. 32w + 31 in fp32, forms the rows of X = K S^T, Y and the output of the
-// chunk's tokens 16w .. 16w + 15, and updates its own columns.  Two LDS exchanges a
-// chunk give every wave what the others formed: the four blocks of Y (for v_new, which
-// every wave forms whole) and the bf16 hi/lo parts of the four column blocks of the
-// state (for the next retrieve).  Each value is produced by the same operations in the
-// same order as in consumer_loop with one 16-row wave, so the results are
-// bit-identical, while the chain of a chunk loses three quarters of the retrieve, Y,
-// the output and the state update.
-//
-// Each exchange buffer is single: a wave rewrites its block of Y (of the state) only
-// after the wait for all four blocks of the other exchange, which every wave signals
-// after its last read of the previous contents.
-template <class V>
-__device__ __forceinline__ void consumer_loop_tsplit(PrefillSmem& sm, const PrefillArgs& p, int64_t s0, int64_t s1,
-                                                     int nchunks, int h, int row0, int wave, int lane0,
-                                                     f32x4 (&S)[2]) {
-  static_assert(V::kTokenSplit && V::VT == 1 && V::NCW == 4, "token-split consumers");
-  const int64_t vstride = int64_t(p.Hv) * D;
-  const int ct = wave;  // this wave's 16-token block and 32-column block
-  const int orow = (16 * ct + (lane0 & 15)) * int(vstride) + 4 * (lane0 >> 4);
-  f32x4* const yx = reinterpret_cast<f32x4*>(sm.Nh);            // Y: [block][lane]
-  uint4* const sx = reinterpret_cast<uint4*>(sm.Nh) + 4 * 64;   // state: [block][hi, lo][lane]
-  // K^T operand base of column blocks 2 ct, 2 ct + 1 (kt_bases with kt / 2 = ct).
-  int ktb;
-  {
-    const int j = lane0 & 15, rl = 4 * (lane0 >> 4) + (j >> 2), sl = kq_sigma(rl);
-    ktb = rl * KSTR + 8 * ((j & 3) ^ (sl & 3)) + 32 * (ct ^ (sl >> 2));
-  }
-  {
-    uint4 Sh, Sl;
-    split_pack(S[0], S[1], Sh, Sl);
-    sx[(2 * ct) * 64 + lane0] = Sh;
-    sx[(2 * ct + 1) * 64 + lane0] = Sl;
-    signal_count(sm, kSx, lane0);
-  }
-  for (int t = 1; t <= nchunks; ++t) {
-    int lane = lane0;
-    asm volatile("" : "+v"(lane));
-    const int g = lane >> 4, n16 = lane & 15;
-    const int64_t cs = s0 + int64_t(t - 1) * C;
-    const int clen = int(s1 - cs < C ? s1 - cs : C);
-    const ChunkBufs cb = chunk_bufs(sm, (t - 1) & 1);
-    // Chunk t - 1 loaded; the state after chunk t - 2 looked at in the same read.
-    const bool sx_ready = wait_count_peek<V::kHooks>(sm, kReady, 4 * t, kSx, 4 * t);
-    uint4 kf[4], qf[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      kf[ks] = frag_kq(cb.K, 16 * ct, ks, lane);
-      qf[ks] = frag_kq(cb.Q, 16 * ct, ks, lane);
-    }
-    if (!sx_ready) wait_count<V::kHooks>(sm, kSx, 4 * t);  // the state after chunk t - 2
-    uint4 Sh[4], Sl[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      Sh[ks] = sx[(2 * ks) * 64 + lane];
-      Sl[ks] = sx[(2 * ks + 1) * 64 + lane];
-    }
-
-    // 1: block ct of X = K S^T and of (Q S^T)^T.
-    f32x4 xk = zero4(), xq = zero4();
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      xk = mfma(kf[ks], Sh[ks], xk);
-      xk = mfma(kf[ks], Sl[ks], xk);
-      xq = mfma(Sh[ks], qf[ks], xq);
-    }
-
-    // 2: Y for rows c = 16ct + 4g + i, as consumer_loop; the output block scaled.
-    {
-      const float4 bc = *reinterpret_cast<const float4*>(cb.bet + 16 * ct + 4 * g);
-      const float4 ec = *reinterpret_cast<const float4*>(cb.eg + 16 * ct + 4 * g);
-      const float b4[4] = {bc.x, bc.y, bc.z, bc.w}, e4[4] = {ec.x, ec.y, ec.z, ec.w};
-      const uint2 vv = read_tr(sm.V + (16 * ct + 4 * g + (n16 >> 2)) * VSTR + vrow<1>(0, 4 * (n16 & 3)));
-      const float vf[4] = {bf16lo_f32(vv.x), bf16hi_f32(vv.x), bf16lo_f32(vv.y), bf16hi_f32(vv.y)};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) xk[i] = b4[i] * (vf[i] - e4[i] * xk[i]);
-      xq = xq * (cb.eg[16 * ct + n16] * p.scale);
-    }
-    signal_count(sm, kVFree, lane);  // V of this chunk read
-    yx[64 * ct + lane] = xk;
-    signal_count(sm, kYx, lane);
-    // T~ (all of it) and this block's P operands, read while the other blocks arrive.
-    uint4 thf[6], tlf[6];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int js = 0; js <= (c >> 1); ++js) {
-        const int i = tile_frag(c, js);
-        thf[i] = tile_row<true>(cb.Th, c, js, lane);
-        tlf[i] = tile_row<true>(cb.Tl, c, js, lane);
-      }
-    const uint4 pq0 = tile_row<true>(cb.P, ct, 0, lane);
-    const uint4 pq1 = tile_row<true>(cb.P, ct, ct >> 1, lane);  // used by ct >= 2 only
-    wait_count<V::kHooks>(sm, kYx, 4 * t);
-    f32x4 Y[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) Y[c] = yx[64 * c + lane];
-
-    // v_new = T~ Y, all 64 rows.
-    uint4 Yh[2], Yl[2];
-#pragma unroll
-    for (int js = 0; js < 2; ++js) split_pack(Y[2 * js], Y[2 * js + 1], Yh[js], Yl[js]);
-    f32x4 Vn[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      Vn[c] = zero4();
-#pragma unroll
-      for (int js = 0; js <= (c >> 1); ++js) {
-        const uint4 th = thf[tile_frag(c, js)], tl = tlf[tile_frag(c, js)];
-        Vn[c] = mfma(th, Yh[js], Vn[c]);
-        Vn[c] = mfma(th, Yl[js], Vn[c]);
-        Vn[c] = mfma(tl, Yh[js], Vn[c]);
-      }
-    }
-
-    // 3: columns 32ct .. 32ct + 31 of S = e^{gamma_last} S + sum_c K[c]^T (d_c v_new[c]).
-    const float dlast = cb.eg[clen - 1];
-    uint4 Uh[2], Ul[2];
-#pragma unroll
-    for (int js = 0; js < 2; ++js) {
-      const float4 d0 = *reinterpret_cast<const float4*>(cb.dd + 32 * js + 4 * g);
-      const float4 d1 = *reinterpret_cast<const float4*>(cb.dd + 32 * js + 16 + 4 * g);
-      const f32x4 e0 = {d0.x, d0.y, d0.z, d0.w}, e1 = {d1.x, d1.y, d1.z, d1.w};
-      split_pack(Vn[2 * js] * e0, Vn[2 * js + 1] * e1, Uh[js], Ul[js]);
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      S[j] = S[j] * dlast;
-#pragma unroll
-      for (int js = 0; js < 2; ++js) {
-        const uint16_t* kp = cb.K + ktb + 32 * js * KSTR + 4 * j;
-        const uint2 a = read_tr(kp), b = read_tr(kp + 16 * KSTR);
-        const uint4 ak = uint4{a.x, a.y, b.x, b.y};
-        S[j] = mfma(ak, Uh[js], S[j]);
-        S[j] = mfma(ak, Ul[js], S[j]);
-      }
-    }
-    signal_count(sm, kConsumed, lane);  // buffers of this chunk no longer read
-    {
-      uint4 h2, l2;
-      split_pack(S[0], S[1], h2, l2);
-      sx[(2 * ct) * 64 + lane] = h2;
-      sx[(2 * ct + 1) * 64 + lane] = l2;
-      signal_count(sm, kSx, lane);
-    }
-
-    // Output block ct: o^T = scale e^gamma (S Q^T) + v_new^T (scale P)^T.
-    xq = mfma(pack_hi(Vn[0], Vn[1]), pq0, xq);
-    if (ct >= 2) xq = mfma(pack_hi(Vn[2], Vn[3]), pq1, xq);
-    // Rows at or past clen fall outside the buffer resource, whose extent ends at the
-    // chunk's last token: the hardware drops their stores (no per-lane branch).
-    {
-      const BufferRsrc orsrc =
-          buffer_rsrc(p.out + cs * vstride + (int64_t(h) * D + row0), uint32_t(clen) * uint32_t(vstride) * 2u);
-      buffer_store8(u32x2{pack_bf16x2(xq[0], xq[1]), pack_bf16x2(xq[2], xq[3])}, orsrc, 2 * orow);
-    }
-  }
-}
-
 // The sequence of rank `rank` in descending length order (ties: lower index
-// first), so the longest chains start first; natural order for large batches.
+// first), so the longest chains start first; natural order for large batches.  `len` and
+// `picked` are LDS scratch (up to kMaxSortedSeqs lengths, and the result).
 template <int NTHREADS>
-__device__ int pick_sequence(PrefillSmem& sm, const PrefillArgs& p, int rank, int tid) {
+__device__ int pick_sequence(int* len, int* picked, const PrefillArgs& p, int rank, int tid) {
   if (p.N <= 1 || p.N > kMaxSortedSeqs) return rank;
-  int* len = reinterpret_cast<int*>(sm.Nh);  // scratch until the first chunk
   for (int i = tid; i < p.N; i += NTHREADS) {
     int64_t a = load_cu(p.cu_seqlens, p.cu_is_64, i), b = load_cu(p.cu_seqlens, p.cu_is_64, i + 1);
     a = a < 0 ? 0 : (a > p.T ? p.T : a);
@@ -2010,10 +1811,10 @@ __device__ int pick_sequence(PrefillSmem& sm, const PrefillArgs& p, int rank, in
       const int lj = len[j];
       r += (lj > li) | ((lj == li) & (j < i));
     }
-    if (r == rank) sm.seq = i;
+    if (r == rank) *picked = i;
   }
   __syncthreads();
-  return sm.seq;
+  return *picked;
 }
 
 // Workgroup b handles slice f of chain `chain` (chain = rank-major, v-head
@@ -2058,7 +1859,7 @@ __global__ __launch_bounds__(V::NTHREADS) void gdn_prefill_kernel(PrefillArgs p)
   const int row0 = V::F == 1 ? 0 : ((bid / 8) % V::F) * V::ROWS;
   if (chain >= p.N * p.Hv) return;  // padding of the last group of 16 chains (workgroup-uniform)
   const int h = chain % p.Hv;
-  const int seq = pick_sequence<NTHREADS>(sm, p, chain / p.Hv, tid);
+  const int seq = pick_sequence<NTHREADS>(reinterpret_cast<int*>(sm.Nh), &sm.seq, p, chain / p.Hv, tid);
   const int hq = h / (p.Hv / p.Hq);
   const int hk = h / (p.Hv / p.Hk);
 
@@ -2112,41 +1913,6 @@ __global__ __launch_bounds__(V::NTHREADS) void gdn_prefill_kernel(PrefillArgs p)
 
   const int64_t state_head = (int64_t(seq) * p.Hv + h) * D * D;
   const int g = lane0 >> 4, n16 = lane0 & 15;
-  if constexpr (V::kTokenSplit) {
-    // Token-split consumers: wave w holds column blocks 2w and 2w + 1 (cols k = 16 kt +
-    // 4g + i) of the slice's rows v = row0 + n16.
-    const int64_t srow = state_head + int64_t(row0 + n16) * D + 32 * wave + 4 * g;
-    f32x4 S2[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if (p.state) {
-        const float4 x = *reinterpret_cast<const float4*>(p.state + srow + 16 * j);
-        S2[j] = f32x4{x.x, x.y, x.z, x.w};
-      } else {
-        S2[j] = zero4();
-      }
-    }
-    if (nchunks > 0) {
-      consumer_loop_tsplit<V>(sm, p, s0, s1, nchunks, h, row0, wave, lane0, S2);
-      if (aborted(sm)) {
-        // A hand-off wait gave up: NaN over the slice's outputs (wave w: tokens
-        // s0 + 16 (4m + w) + n16) and state.
-        const int64_t vstride = int64_t(p.Hv) * D;
-        uint16_t* obase = p.out + int64_t(h) * D + row0 + 4 * (lane0 >> 4);
-        for (int64_t tok = s0 + 16 * wave + n16; tok < s1; tok += 64)
-          *reinterpret_cast<uint2*>(obase + tok * vstride) = uint2{kNaNx2, kNaNx2};
-        const float nan = __builtin_nanf("");
-        S2[0] = S2[1] = f32x4{nan, nan, nan, nan};
-      }
-    }
-    if (nchunks > 0 || p.state != p.new_state) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        *reinterpret_cast<float4*>(p.new_state + srow + 16 * j) = make_float4(S2[j][0], S2[j][1], S2[j][2], S2[j][3]);
-    }
-    return;
-  }
-
   // Consumer state slab: rows v = row0 + VW*wave + vrow(vt, n16), cols k = 16*kt + 4g + i.
   f32x4 S[VT][8];
 #pragma unroll
@@ -2421,8 +2187,7 @@ __global__ __launch_bounds__(V::NTHREADS) void gdn_prefill_persistent_kernel(Pre
 }
 
 // ---------------------------------------------------------------------------
-// Prep kernel of the two-kernel path: T~, P and the gates of every chunk-head, one
-// wave each.
+// State pass of the two-kernel path
 // ---------------------------------------------------------------------------
 
 // Rows 16 I + lane%16 of a chunk's K or Q slice (stride: bytes from token to token) as
@@ -2450,6 +2215,398 @@ struct RowFrags {
       }
   }
 };
+
+// LDS of the state pass.
+struct __align__(16) StateSmem {
+  uint16_t K[2][C * KSTR];               // K chunk [c][perm(k)], by chunk parity
+  uint16_t T[2][8 * 2 * kTileUnits1];    // T~ hi, T~ lo: image fragments
+  float gate[2][3 * C];                  // beta, e^gamma, e^{gamma_last - gamma}
+  uint16_t V[2][C * 16];                 // V slice [token][state row]
+  uint4 Y[4][64];                        // exchange: Y, 16-token blocks [block][lane]: hi, lo
+  uint4 S[3][4][2][64];                  // exchange: state, 32-column blocks [block][hi, lo][lane]
+  uint2 Vn[2][4][64];                    // v_new (hi parts), 16-token blocks [block][lane]
+  int sync[16];                          // hand-off counters
+  int seq;
+};
+static_assert(sizeof(StateSmem) <= 160 * 1024);
+
+// Hand-offs of the state pass.  kAbort as in the other kernels.  "Loaded" and "output read"
+// count by chunk parity: a helper wave may be a chunk ahead of another, and with one counter
+// its signal could stand in for the other's.
+enum StateCounter {
+  kLoaded = 0,     // + parity: a helper wave stored its part of the chunk (4 a chunk)
+  kChunkRead = 2,  // a consumer wave has read the chunk's buffers (4 a chunk)
+  kStateIn = 3,        // a consumer wave stored its state columns (4 a chunk, 4 at start)
+  kYIn = 5,        // a consumer wave stored its block of Y (4 a chunk)
+  kVnewIn = 6,         // a consumer wave stored its block of v_new (4 a chunk)
+  kOutRead = 7     // + parity: a helper wave has read the chunk's state and v_new (4 a chunk)
+};
+static_assert(kAbort == 4, "kAbort between the state pass's counters");
+
+// What a helper thread moves of a chunk: K (four 16-byte units), T~ (three), gates and V.
+struct StateLoad {
+  u32x4 k[4], t[3], g, v;
+};
+
+constexpr int kStateLoaders = 256;  // helper threads (four waves)
+
+// The helper waves keep off the chain whatever the state recurrence does not need.  Wave w
+// * loads (its quarter of) K, T~, the gates and the V slice of chunk t into the LDS buffers
+//   of parity t & 1 once the consumers are done with chunk t - 2.  The loads go two chunks
+//   ahead (two register sets) and are unconditional (rows past the chunk lie outside the
+//   buffer and read as zeros), so the compiler waits for exactly the older set;
+// * forms and stores the output of the chunk's tokens 16w .. 16w + 15, from the chunk-start
+//   state (hi parts) and v_new of the consumers' exchanges and its own Q rows and P
+//   fragments, which no other wave reads: they go straight into registers.
+// A wave that issues loads while the memory queue is full stalls (about 800 cycles a chunk);
+// here that delays no consumer.
+__device__ __forceinline__ void state_helper(StateSmem& sm, const PrefillArgs& p, const u32x4* tiles, int64_t s0,
+                                             int64_t s1, int nchunks, int h, int hq, int hk, int row0, int w,
+                                             int lane0) {
+  const int pt = 64 * w + lane0;
+  const int ct = w;  // this wave's 16-token output block
+  const int64_t vstride = int64_t(p.Hv) * D;
+  const int kstr = p.Hk * D * 2, qstr = p.Hq * D * 2, vstr = p.Hv * D * 2;
+  const int koff = (pt >> 4) * kstr + 16 * (pt & 15);
+  const int voff = ((pt >> 1) & 63) * vstr + 16 * (pt & 1);
+  const int goff = kTileUnits + min(pt, kGateUnits - 1);
+  const int orow = (16 * ct + (lane0 & 15)) * int(vstride) + 4 * (lane0 >> 4);
+  auto chunk_len = [&](int64_t cs) { return int(s1 - cs < C ? s1 - cs : C); };
+  auto load = [&](int t, StateLoad& r) {
+    const int64_t cs = s0 + int64_t(t) * C;
+    const int clen = chunk_len(cs);
+    const BufferRsrc kr = buffer_rsrc(const_cast<uint16_t*>(p.k) + (cs * p.Hk + hk) * D, uint32_t(clen - 1) * kstr + 2 * D);
+    const BufferRsrc vr =
+        buffer_rsrc(const_cast<uint16_t*>(p.v) + (cs * p.Hv + h) * D + row0, uint32_t(clen - 1) * vstr + 32);
+    const u32x4* im = tiles + int64_t(t) * p.Hv * kTileImage;
+#pragma unroll
+    for (int it = 0; it < 4; ++it) r.k[it] = __builtin_amdgcn_raw_buffer_load_b128(kr, koff + 16 * it * kstr, 0, 0);
+#pragma unroll
+    for (int it = 0; it < 3; ++it) r.t[it] = im[pt + kStateLoaders * it];
+    r.g = im[goff];
+    r.v = __builtin_amdgcn_raw_buffer_load_b128(vr, voff, 0, 0);
+  };
+  auto stage = [&](int t, StateLoad& r, int lane) {
+    const int b = t & 1;
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const int c = (pt >> 4) + 16 * it, sg = pt & 15;
+      const int col0 = (8 * sg) & ~31, r0 = (8 * sg) & 31;
+      *reinterpret_cast<uint2*>(sm.K[b] + kq_off(c, col0 + perm32(r0))) = uint2{r.k[it][0], r.k[it][1]};
+      *reinterpret_cast<uint2*>(sm.K[b] + kq_off(c, col0 + perm32(r0 + 4))) = uint2{r.k[it][2], r.k[it][3]};
+    }
+#pragma unroll
+    for (int it = 0; it < 3; ++it) *reinterpret_cast<u32x4*>(sm.T[b] + 8 * (pt + kStateLoaders * it)) = r.t[it];
+    if (pt < kGateUnits) *reinterpret_cast<u32x4*>(sm.gate[b] + 4 * pt) = r.g;
+    if (pt < 2 * C) *reinterpret_cast<u32x4*>(sm.V[b] + 8 * pt) = r.v;
+    signal_count(sm, kLoaded + b, lane);
+  };
+  // The output block's own operands: Q rows, P fragments and e^gamma of its tokens.
+  RowFrags qf;
+  u32x4 pf[2];
+  float eo;
+  auto load_out = [&](int t, int lane) {
+    const int64_t cs = s0 + int64_t(t) * C;
+    qf.load(buffer_rsrc(const_cast<uint16_t*>(p.q) + (cs * p.Hq + hq) * D, uint32_t(chunk_len(cs) - 1) * qstr + 2 * D),
+            qstr, ct, lane);
+    const u32x4* im = tiles + int64_t(t) * p.Hv * kTileImage;
+    pf[0] = im[2 * kTileUnits1 + 64 * tile_frag(ct, 0) + lane];
+    pf[1] = im[2 * kTileUnits1 + 64 * tile_frag(ct, ct >> 1) + lane];  // used by ct >= 2 only
+    eo = reinterpret_cast<const float*>(im + kTileUnits)[C + 16 * ct + (lane & 15)];
+  };
+  // o^T = scale e^gamma (S Q^T) + v_new^T (scale P)^T of chunk t, tokens 16 ct .. +15.
+  auto output = [&](int t, int sbuf, int lane) {
+    wait_count<false>(sm, kVnewIn, 4 * (t + 1));
+    uint4 Sh[4];
+    uint2 vn[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) Sh[ks] = sm.S[sbuf][ks][0][lane];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) vn[c] = sm.Vn[t & 1][c][lane];
+    signal_count(sm, kOutRead + (t & 1), lane);
+    qf.to_kappa();
+    f32x4 o = zero4();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) o = mfma(Sh[ks], __builtin_bit_cast(uint4, qf.v[ks]), o);
+    o = o * (eo * p.scale);
+    o = mfma(uint4{vn[0].x, vn[0].y, vn[1].x, vn[1].y}, __builtin_bit_cast(uint4, pf[0]), o);
+    if (ct >= 2) o = mfma(uint4{vn[2].x, vn[2].y, vn[3].x, vn[3].y}, __builtin_bit_cast(uint4, pf[1]), o);
+    // Rows at or past the chunk's end fall outside the buffer: the hardware drops their
+    // stores (no per-lane branch).
+    const int64_t cs = s0 + int64_t(t) * C;
+    buffer_store8(u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])},
+                  buffer_rsrc(p.out + cs * vstride + (int64_t(h) * D + row0),
+                              uint32_t(chunk_len(cs)) * uint32_t(vstride) * 2u),
+                  2 * orow);
+  };
+  StateLoad ra, rb;
+  const int last = nchunks - 1;
+  load(0, ra);
+  load(min(1, last), rb);
+  load_out(0, lane0);
+  stage(0, ra, lane0);
+  load(min(2, last), ra);
+  if (last >= 1) stage(1, rb, lane0);
+  load(min(3, last), rb);
+  int sbuf = 0;  // t % 3
+  auto tick = [&](int t, StateLoad& r) {
+    int lane = lane0;
+    asm volatile("" : "+v"(lane));
+    // Chunk t + 2 first: the consumers take it sooner than they miss this output.
+    if (t + 2 <= last) {
+      wait_count<false>(sm, kChunkRead, 4 * (t + 1));
+      stage(t + 2, r, lane);
+    }
+    output(t, sbuf, lane);
+    sbuf = sbuf == 2 ? 0 : sbuf + 1;
+    load_out(min(t + 1, last), lane);
+    load(min(t + 4, last), r);
+  };
+  for (int t = 0; t <= last; t += 2) {
+    tick(t, ra);
+    if (t + 1 <= last) tick(t + 1, rb);
+  }
+}
+
+// The four consumer waves share the slice's 16 state rows: wave w keeps state columns
+// 32w .. 32w + 31 in fp32, forms the rows of X = K S^T and Y of the chunk's tokens
+// 16w .. 16w + 15, and updates its own columns.  Two LDS exchanges a chunk give every wave
+// what the others formed: the four blocks of Y (for v_new, which every wave forms whole)
+// and the bf16 hi/lo parts of the four column blocks of the state (for the next retrieve).
+// Each value is produced by the same operations in the same order as in consumer_loop, so
+// the results are those of the one-kernel path bit for bit.
+//
+// The chain of a chunk is LDS round trips and short dependent products (about 2.6k cycles,
+// 1.3 us, a chunk), so every other operand is read where the wave computes or waits anyway:
+// T~ behind the state, under the retrieve; the update's behind Y, under v_new; the next
+// chunk's K rows, gates and V after the state is stored, while the other waves store theirs
+// (under v_new they would hold up its first operands).  A wave splits its block of Y into
+// bf16 hi and lo before the exchange, so that no wave splits all four.
+//
+// A wave rewrites its block of Y only after the wait for all four blocks of the state,
+// which every wave signals after its last read of Y.  The state (three buffers) and v_new
+// (two) are also read by the helpers, up to a chunk later.
+//
+// One 4,096-token sequence at 32 v-heads (256 workgroups, 64 chunks each), inputs from HBM,
+// prep kernel included: 108 us a call; with K, Q, T~ and P all staged through the LDS and the
+// outputs formed by the consumers 121.5; with the consumers loading their own K, Q and P
+// rows into registers 152 (their loads stall behind the loaders').
+__device__ __forceinline__ void state_consumer(StateSmem& sm, const PrefillArgs& p, int64_t s0, int64_t s1, int nchunks,
+                                               int wave, int lane0, f32x4 (&S)[2]) {
+  const int ct = wave;  // this wave's 16-token block and 32-column block
+  // K^T operand base of column blocks 2 ct, 2 ct + 1 (kt_bases with kt / 2 = ct).
+  int ktb;
+  {
+    const int j = lane0 & 15, rl = 4 * (lane0 >> 4) + (j >> 2), sl = kq_sigma(rl);
+    ktb = rl * KSTR + 8 * ((j & 3) ^ (sl & 3)) + 32 * (ct ^ (sl >> 2));
+  }
+  // What the retrieve and Y of a chunk take besides the state, read a chunk ahead.
+  uint4 kf[4];
+  f32x4 b4, e4;
+  uint2 vv;
+  auto read_ahead = [&](int t, int lane) {
+    const int b = t & 1, g = lane >> 4, n16 = lane & 15;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) kf[ks] = frag_kq(sm.K[b], 16 * ct, ks, lane);
+    b4 = ld4(sm.gate[b] + 16 * ct + 4 * g);
+    e4 = ld4(sm.gate[b] + C + 16 * ct + 4 * g);
+    vv = read_tr(sm.V[b] + (16 * ct + 4 * g + (n16 >> 2)) * 16 + 4 * (n16 & 3));
+  };
+  auto put_state = [&](int sbuf, int lane) {
+    uint4 Sh, Sl;
+    split_pack(S[0], S[1], Sh, Sl);
+    sm.S[sbuf][ct][0][lane] = Sh;
+    sm.S[sbuf][ct][1][lane] = Sl;
+    signal_count(sm, kStateIn, lane);
+  };
+  put_state(0, lane0);
+  wait_count<false>(sm, kLoaded, 4);
+  read_ahead(0, lane0);
+  int sbuf = 0;  // t % 3
+  for (int t = 0; t < nchunks; ++t) {
+    int lane = lane0;
+    asm volatile("" : "+v"(lane));
+    const int g = lane >> 4;
+    const int64_t cs = s0 + int64_t(t) * C;
+    const int clen = int(s1 - cs < C ? s1 - cs : C);
+    const int b = t & 1;
+    // The chunk-start state; the next chunk's buffers looked at in the same read (the last
+    // chunk looks at its own).
+    const int tn = min(t + 1, nchunks - 1);
+    const bool loaded = wait_count_peek<false>(sm, kStateIn, 4 * (t + 1), kLoaded + (tn & 1), 4 * ((tn >> 1) + 1));
+    uint4 Sh[4], Sl[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      Sh[ks] = sm.S[sbuf][ks][0][lane];
+      Sl[ks] = sm.S[sbuf][ks][1][lane];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    uint4 thf[kTileFrags], tlf[kTileFrags];  // T~
+#pragma unroll
+    for (int i = 0; i < kTileFrags; ++i) {
+      thf[i] = *reinterpret_cast<const uint4*>(sm.T[b] + 8 * (64 * i + lane));
+      tlf[i] = *reinterpret_cast<const uint4*>(sm.T[b] + 8 * (kTileUnits1 + 64 * i + lane));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // 1: block ct of X = K S^T; Y for rows c = 16ct + 4g + i, as consumer_loop.
+    f32x4 xk = zero4();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      xk = mfma(kf[ks], Sh[ks], xk);
+      xk = mfma(kf[ks], Sl[ks], xk);
+    }
+    {
+      const float vf[4] = {bf16lo_f32(vv.x), bf16hi_f32(vv.x), bf16lo_f32(vv.y), bf16hi_f32(vv.y)};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xk[i] = b4[i] * (vf[i] - e4[i] * xk[i]);
+    }
+    {
+      uint2 hi, lo;
+      split4(xk, hi, lo);
+      sm.Y[ct][lane] = uint4{hi.x, hi.y, lo.x, lo.y};
+    }
+    signal_count(sm, kYIn, lane);
+    // All of Y; the helpers done with the v_new (of chunk t - 2) and the state (before it)
+    // whose buffers this chunk rewrites, looked at in the same read.
+    const bool out_read = wait_count_peek<false>(sm, kYIn, 4 * (t + 1), kOutRead + b, 4 * (t >> 1));
+    uint4 Y[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) Y[c] = sm.Y[c][lane];
+    __builtin_amdgcn_sched_barrier(0);
+    // The update's operands: its decays and K^T (columns 32ct .. +31).
+    const float dlast = sm.gate[b][C + clen - 1];
+    f32x4 ed[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) ed[c] = ld4(sm.gate[b] + 2 * C + 16 * c + 4 * g);
+    uint4 kt[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int js = 0; js < 2; ++js) {
+        const uint16_t* kp = sm.K[b] + ktb + 32 * js * KSTR + 4 * j;
+        const uint2 k0 = read_tr(kp), k1 = read_tr(kp + 16 * KSTR);
+        kt[j][js] = uint4{k0.x, k0.y, k1.x, k1.y};
+      }
+    // What the next chunk's retrieve and Y take besides the state.
+    signal_count(sm, kChunkRead, lane);  // buffers of this chunk no longer read
+    __builtin_amdgcn_sched_barrier(0);
+
+    // 2: v_new = T~ Y, all 64 rows; this wave's block of it (hi parts) to the helpers.
+    uint4 Yh[2], Yl[2];
+#pragma unroll
+    for (int js = 0; js < 2; ++js) {
+      Yh[js] = uint4{Y[2 * js].x, Y[2 * js].y, Y[2 * js + 1].x, Y[2 * js + 1].y};
+      Yl[js] = uint4{Y[2 * js].z, Y[2 * js].w, Y[2 * js + 1].z, Y[2 * js + 1].w};
+    }
+    f32x4 Vn[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      Vn[c] = zero4();
+#pragma unroll
+      for (int js = 0; js <= (c >> 1); ++js) {
+        const uint4 th = thf[tile_frag(c, js)], tl = tlf[tile_frag(c, js)];
+        Vn[c] = mfma(th, Yh[js], Vn[c]);
+        Vn[c] = mfma(th, Yl[js], Vn[c]);
+        Vn[c] = mfma(tl, Yh[js], Vn[c]);
+      }
+    }
+    if (!out_read) wait_count<false>(sm, kOutRead + b, 4 * (t >> 1));
+
+    // 3: columns 32ct .. 32ct + 31 of S = e^{gamma_last} S + sum_c K[c]^T (d_c v_new[c]).
+    uint4 Uh[2], Ul[2];
+#pragma unroll
+    for (int js = 0; js < 2; ++js) split_pack(Vn[2 * js] * ed[2 * js], Vn[2 * js + 1] * ed[2 * js + 1], Uh[js], Ul[js]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      S[j] = S[j] * dlast;
+#pragma unroll
+      for (int js = 0; js < 2; ++js) {
+        S[j] = mfma(kt[j][js], Uh[js], S[j]);
+        S[j] = mfma(kt[j][js], Ul[js], S[j]);
+      }
+    }
+    sbuf = sbuf == 2 ? 0 : sbuf + 1;
+    put_state(sbuf, lane);
+    const f32x4 v = ct == 0 ? Vn[0] : ct == 1 ? Vn[1] : ct == 2 ? Vn[2] : Vn[3];
+    sm.Vn[b][ct][lane] = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    signal_count(sm, kVnewIn, lane);
+    if (t + 1 < nchunks) {
+      if (!loaded) wait_count<false>(sm, kLoaded + (tn & 1), 4 * ((tn >> 1) + 1));
+      read_ahead(tn, lane);
+    }
+  }
+}
+
+// Workgroup b handles slice f (16 state rows) of chain `chain` (rank-major, v-head minor),
+// placed as in gdn_prefill_kernel with F = 8: the slices of a GQA pair of chains share an
+// XCD.  Waves 0-3 are consumers, 4-7 loaders.
+constexpr int kStateSlices = 8;
+__global__ __launch_bounds__(512) void gdn_prefill_state_kernel(PrefillArgs p) {
+  constexpr int F = kStateSlices;
+  __shared__ StateSmem sm;
+  const int tid = threadIdx.x;
+  const int lane0 = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bid = blockIdx.x;
+  const int chain = (bid / (16 * F)) * 16 + 2 * (bid % 8) + (bid / 8) % (2 * F) / F;
+  const int row0 = ((bid / 8) % F) * 16;
+  if (chain >= p.N * p.Hv) return;  // padding of the last group of 16 chains (workgroup-uniform)
+  const int h = chain % p.Hv;
+  const int seq = pick_sequence<512>(reinterpret_cast<int*>(sm.K), &sm.seq, p, chain / p.Hv, tid);
+  const int hq = h / (p.Hv / p.Hq);
+  const int hk = h / (p.Hv / p.Hk);
+  const SeqRange sr = seq_range(p, seq);
+  const int64_t s0 = sr.s0, s1 = sr.s1;
+  const int nchunks = int((s1 - s0 + C - 1) / C);
+  if (tid < 16) sm.sync[tid] = 0;
+  __syncthreads();  // counters cleared; pick_sequence's scratch read
+  const u32x4* tiles =
+      reinterpret_cast<const u32x4*>(p.tiles) + (int64_t(chunks_before(p, seq, lane0)) * p.Hv + h) * kTileImage;
+
+  if (wave >= 4) {
+    if (nchunks > 0) {
+      state_helper(sm, p, tiles, s0, s1, nchunks, h, hq, hk, row0, wave - 4, lane0);
+      if (aborted(sm)) {
+        // A hand-off wait gave up: NaN over the slice's outputs (wave w: tokens
+        // s0 + 16 (4m + w) + lane % 16).
+        const int64_t vstride = int64_t(p.Hv) * D;
+        uint16_t* obase = p.out + int64_t(h) * D + row0 + 4 * (lane0 >> 4);
+        for (int64_t tok = s0 + 16 * (wave - 4) + (lane0 & 15); tok < s1; tok += 64)
+          *reinterpret_cast<uint2*>(obase + tok * vstride) = uint2{kNaNx2, kNaNx2};
+      }
+    }
+    return;
+  }
+
+  // Wave w holds column blocks 2w and 2w + 1 (cols k = 16 kt + 4g + i) of the slice's
+  // rows v = row0 + n16.
+  const int g = lane0 >> 4, n16 = lane0 & 15;
+  const int64_t srow = (int64_t(seq) * p.Hv + h) * D * D + int64_t(row0 + n16) * D + 32 * wave + 4 * g;
+  f32x4 S[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    S[j] = zero4();
+    if (p.state) S[j] = ld4(p.state + srow + 16 * j);
+  }
+  if (nchunks > 0) {
+    state_consumer(sm, p, s0, s1, nchunks, wave, lane0, S);
+    if (aborted(sm)) {  // a hand-off wait gave up: NaN over the slice's state
+      const float nan = __builtin_nanf("");
+      S[0] = S[1] = f32x4{nan, nan, nan, nan};
+    }
+  }
+  if (nchunks > 0 || p.state != p.new_state) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      *reinterpret_cast<float4*>(p.new_state + srow + 16 * j) = make_float4(S[j][0], S[j][1], S[j][2], S[j][3]);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Prep kernel of the two-kernel path: T~, P and the gates of every chunk-head, one
+// wave each.
+// ---------------------------------------------------------------------------
 
 __device__ __forceinline__ f32x4 row_product(const RowFrags& a, const RowFrags& b) {
   f32x4 acc = zero4();
@@ -2887,8 +3044,6 @@ int64_t prefill_work_items(int64_t chains) {
 namespace {
 // Largest workspace the two-kernel path uses; bigger batches take one kernel.
 constexpr int64_t kMaxWorkspaceBytes = int64_t(2) << 30;
-// Images above this size are read back mostly from HBM by the state pass.
-constexpr int64_t kDeepImageBytes = int64_t(64) << 20;
 }  // namespace
 
 // Batches split 4 or 8 ways repeat the producer work in every slice of a chain and
@@ -2928,15 +3083,14 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream, hipEvent_t d
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (F == 4) return launch_variant<Variant<2, 1, false, true>>(a, stream, done);
-    // Split 8 ways, images beyond what the caches keep between the two kernels are
-    // loaded two chunks ahead (one sequence, 32 v-heads, 19,200-byte images: 12,288
-    // tokens, 118 MB of images, 420.1 -> 396.9 us; 10,500 tokens 349.8 -> 333.8;
-    // 8,192 tokens, 79 MB, 255.7 -> 252.5; 6,000 tokens, 58 MB, 187.8 -> 188.0).
-    // Split 4 ways it measured no change (two 4,096-token sequences, images of whole
-    // tiles: 186.2 -> 185.8 us).
-    if (prefill_workspace_bytes(a.N, a.T, a.Hv) > kDeepImageBytes)
-      return launch_variant<Variant<4, 1, false, true, 4, false, true, true>>(a, stream, done);
-    return launch_variant<Variant<4, 1, false, true, 4, false, true>>(a, stream, done);
+    const int64_t chains = int64_t(a.N) * a.Hv;
+    const dim3 sgrid(unsigned((chains + 15) / 16 * 16 * kStateSlices)), sblock(512);
+    if (done != nullptr) {
+      hipExtLaunchKernelGGL(gdn_prefill_state_kernel, sgrid, sblock, 0, stream, nullptr, done, 0, a);
+    } else {
+      hipLaunchKernelGGL(gdn_prefill_state_kernel, sgrid, sblock, 0, stream, a);
+    }
+    return hipGetLastError();
   }
   // Split chains use 16-row consumer waves (VT = 1), whose per-chunk chain is
   // shorter than a 32-row wave's.  Unsplit chains (F = 1) keep four 32-row waves:
