@@ -47,7 +47,10 @@ struct PrefillArgs {
   // Two-kernel path: workspace of prefill_workspace_bytes(...) bytes for the
   // prepared T~/P tiles; null (or a batch that the single kernel serves) => one kernel.
   uint16_t* tiles;
-  int prep_slots;           // set by the launcher: most chunks of a batch with valid offsets
+  // Set by the launcher of the two-kernel path: the most chunks a launch with valid offsets
+  // covers, and the launch's window of each sequence (win_tokens = 0: all of it).
+  int prep_slots;
+  int64_t win_begin, win_tokens;
 };
 
 // Workspace bytes of the two-kernel prefill path for these sizes on the current
@@ -86,8 +89,9 @@ hipError_t prefill_scratch(void** ptr);
 
 // The drop-in gdn_prefill's launcher: launch_prefill, except that a batch of few
 // chains whose sequences average at least kDropinTwoKernelTokens tokens runs the
-// two-kernel path in a per-device scratch of the library (kPrefillDropinScratchBytes)
-// when its images fit, ordered between launches by an event.
+// two-kernel path in a per-device scratch of the library (kPrefillDropinScratchBytes),
+// in windows of the sequences if its images do not fit, ordered between launches by an
+// event.
 constexpr int64_t kPrefillDropinScratchBytes = int64_t(128) << 20;
 constexpr int64_t kDropinTwoKernelTokens = 1024;
 hipError_t launch_prefill_dropin(const PrefillArgs& args, hipStream_t stream);

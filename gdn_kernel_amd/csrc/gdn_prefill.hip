@@ -372,7 +372,8 @@ __device__ __forceinline__ int64_t load_cu(const void* cu, int is64, int i) {
   return is64 ? static_cast<const int64_t*>(cu)[i] : int64_t(static_cast<const int32_t*>(cu)[i]);
 }
 
-// Tokens [s0, s1) of sequence i, its offsets clamped into [0, T].
+// Tokens [s0, s1) of sequence i, its offsets clamped into [0, T]; two-kernel path: of the
+// launch's window of it (win_tokens tokens from win_begin on; 0 = the whole sequence).
 struct SeqRange {
   int64_t s0, s1;
 };
@@ -380,6 +381,11 @@ __device__ __forceinline__ SeqRange seq_range(const PrefillArgs& p, int i) {
   int64_t a = load_cu(p.cu_seqlens, p.cu_is_64, i), b = load_cu(p.cu_seqlens, p.cu_is_64, i + 1);
   a = a < 0 ? 0 : (a > p.T ? p.T : a);
   b = b < a ? a : (b > p.T ? p.T : b);
+  if (p.win_tokens > 0) {
+    a += p.win_begin;
+    a = a < b ? a : b;
+    b = b - a < p.win_tokens ? b : a + p.win_tokens;
+  }
   return SeqRange{a, b};
 }
 
@@ -1863,10 +1869,17 @@ __global__ __launch_bounds__(V::NTHREADS) void gdn_prefill_kernel(PrefillArgs p)
   const int hq = h / (p.Hv / p.Hq);
   const int hk = h / (p.Hv / p.Hk);
 
-  int64_t s0 = load_cu(p.cu_seqlens, p.cu_is_64, seq);
-  int64_t s1 = load_cu(p.cu_seqlens, p.cu_is_64, seq + 1);
-  s0 = s0 < 0 ? 0 : (s0 > p.T ? p.T : s0);
-  s1 = s1 < s0 ? s0 : (s1 > p.T ? p.T : s1);
+  int64_t s0, s1;
+  if constexpr (V::kLoad) {
+    const SeqRange r = seq_range(p, seq);
+    s0 = r.s0;
+    s1 = r.s1;
+  } else {
+    s0 = load_cu(p.cu_seqlens, p.cu_is_64, seq);
+    s1 = load_cu(p.cu_seqlens, p.cu_is_64, seq + 1);
+    s0 = s0 < 0 ? 0 : (s0 > p.T ? p.T : s0);
+    s1 = s1 < s0 ? s0 : (s1 > p.T ? p.T : s1);
+  }
   const int nchunks = int((s1 - s0 + C - 1) / C);
 
   if (nchunks > 0) {
@@ -2894,7 +2907,10 @@ OrderedScratch g_no_alloc[kMaxDevices];
 // again as it completes.  If the launch fails after the prep kernel was enqueued,
 // the event is recorded behind it all the same, so the next launch still waits for
 // the orphaned kernel.
-hipError_t launch_ordered(const PrefillArgs& a, hipStream_t stream, OrderedScratch* table, const void* symbol) {
+hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t slots, hipEvent_t done);
+
+hipError_t launch_ordered(const PrefillArgs& a, hipStream_t stream, OrderedScratch* table, const void* symbol,
+                          int64_t bytes) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
@@ -2915,7 +2931,8 @@ hipError_t launch_ordered(const PrefillArgs& a, hipStream_t stream, OrderedScrat
   }
   PrefillArgs b = a;
   b.tiles = static_cast<uint16_t*>(d.addr);
-  e = launch_prefill(b, stream, d.done);  // the state pass records `done` as it completes
+  // The (last) state pass records `done` as it completes.
+  e = launch_two_kernels(b, stream, bytes / (int64_t(a.Hv) * kTileImage * 16), d.done);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     (void)hipEventRecord(d.done, stream);
@@ -2957,24 +2974,26 @@ int64_t prefill_static_device_bytes() {
 // The drop-in gdn_prefill.  A batch of N sequences averaging at least
 // kDropinTwoKernelTokens tokens (T >= kDropinTwoKernelTokens N), whose chains the
 // launcher splits 4 or 8 ways, runs on the two-kernel path (each chunk prepared once)
-// in dropin_scratch when its images fit; everything else, and any launch on a stream
-// that is being captured into a graph, runs launch_prefill as is.  (The host sees N
+// in dropin_scratch, in windows if its images do not fit; everything else, and any launch
+// on a stream that is being captured into a graph, runs launch_prefill as is.  (The host sees N
 // and T, not the lengths; measured, one kernel against two, µs: [2048, 2048] 111.2 /
 // 99.2, [300, 4000] 189.4 / 150.2, [1000, 1100] 62.2 / 59.8, [900, 1200, 100, 3000]
 // at 16 v-heads 142.2 / 114.0, and below the threshold [600, 700] 42.5 / 42.4,
 // [512] x 4 at 16 v-heads 32.7 / 36.9.)  Launches on the scratch are ordered on the
 // device (launch_ordered), so calls on any streams stay correct, and calls on one
 // stream wait for nothing they would not wait for anyway.
+namespace {
+int split_factor(int64_t chains);
+}
 hipError_t launch_prefill_dropin(const PrefillArgs& a, hipStream_t stream) {
-  const int64_t need =
-      a.N >= 1 && a.T >= kDropinTwoKernelTokens * a.N ? prefill_workspace_bytes(a.N, a.T, a.Hv) : 0;
-  if (need <= 0 || need > kPrefillDropinScratchBytes || a.spin_limit != 0 || a.ready_chunks != 0 ||
+  // (Room for at least one chunk a sequence: N Hv <= 64 images, see split_factor.)
+  if (a.T < kDropinTwoKernelTokens * a.N || split_factor(int64_t(a.N) * a.Hv) < 4 || a.spin_limit != 0 || a.ready_chunks != 0 ||
       a.aborts != nullptr || a.tiles != nullptr)
     return launch_prefill(a, stream);
   hipError_t e = hipSuccess;
   if (stream_capturing(stream, &e)) return launch_prefill(a, stream);
   if (e != hipSuccess) return e;
-  return launch_ordered(a, stream, g_dropin, HIP_SYMBOL(dropin_scratch));
+  return launch_ordered(a, stream, g_dropin, HIP_SYMBOL(dropin_scratch), kPrefillDropinScratchBytes);
 }
 
 // gdn_prefill_no_alloc: the two-kernel path in `scratch` for batches that take it.
@@ -2994,7 +3013,7 @@ hipError_t launch_prefill_no_alloc(const PrefillArgs& a, hipStream_t stream) {
     return launch_prefill(b, stream);
   }
   if (e != hipSuccess) return e;
-  return launch_ordered(a, stream, g_no_alloc, HIP_SYMBOL(scratch));
+  return launch_ordered(a, stream, g_no_alloc, HIP_SYMBOL(scratch), kPrefillScratchBytes);
 }
 
 // Reads (and with `reset` clears) this device's give-up count, after
@@ -3060,6 +3079,52 @@ int64_t prefill_workspace_bytes(int N, int64_t T, int Hv) {
   return bytes <= kMaxWorkspaceBytes ? bytes : 0;
 }
 
+namespace {
+// The two-kernel path with room for `slots` chunk images a v-head (at least N).  If the
+// chunks that any offsets can give do not fit (one or two sequences cannot overlap: at most
+// ceil(T / C) + N - 1; more, if malformed, can: N ceil(T / C)), the batch runs in windows of
+// equally many chunks of every sequence, each a prep kernel and a state pass that takes the
+// state up where the window before left it, in new_state: the same operations in the same
+// order.  A window costs about 8 us (the launches, and both kernels filling and draining
+// the chip); one 16,384-token sequence at 32 v-heads takes 412 us in two windows, 598 in one
+// kernel.
+hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t slots, hipEvent_t done) {
+  const int64_t tc = (a.T + C - 1) / C;
+  const int64_t most = a.N <= 2 ? tc + a.N - 1 : a.N * tc;  // chunks any offsets can give
+  const int64_t fit = most <= slots ? tc : slots / a.N;     // chunks of a sequence a window
+  const int64_t windows = (tc + fit - 1) / fit, w = (tc + windows - 1) / windows;
+  // Valid offsets give at most T / C + N chunks.
+  PrefillArgs b = a;
+  b.prep_slots = int(tc + a.N - 1 < a.N * w ? tc + a.N - 1 : a.N * w);
+  const int64_t chains = int64_t(a.N) * a.Hv;
+  for (int64_t i = 0; i < windows; ++i) {
+    if (windows > 1) {
+      b.win_begin = i * w * C;
+      b.win_tokens = w * C;
+    }
+    const int64_t grid = (int64_t(b.prep_slots) * a.Hv + kPrepWaves - 1) / kPrepWaves;
+    hipLaunchKernelGGL(gdn_prefill_prep_kernel, dim3(unsigned(grid)), dim3(64 * kPrepWaves), 0, stream, b);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const hipEvent_t last = i + 1 == windows ? done : nullptr;
+    if (split_factor(chains) == 4) {
+      e = launch_variant<Variant<2, 1, false, true>>(b, stream, last);
+    } else {
+      const dim3 sgrid(unsigned((chains + 15) / 16 * 16 * kStateSlices)), sblock(512);
+      if (last != nullptr) {
+        hipExtLaunchKernelGGL(gdn_prefill_state_kernel, sgrid, sblock, 0, stream, nullptr, last, 0, b);
+      } else {
+        hipLaunchKernelGGL(gdn_prefill_state_kernel, sgrid, sblock, 0, stream, b);
+      }
+      e = hipGetLastError();
+    }
+    if (e != hipSuccess) return e;
+    b.state = a.new_state;
+  }
+  return hipSuccess;
+}
+}  // namespace
+
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream, hipEvent_t done) {
   const int F = split_factor(int64_t(a.N) * a.Hv);
   // Launches that use the testing hooks get kernels with the hooks compiled in;
@@ -3073,25 +3138,8 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream, hipEvent_t d
       default: return launch_variant<SplitVariant8<true>>(a, stream);
     }
   }
-  if (a.tiles != nullptr && prefill_workspace_bytes(a.N, a.T, a.Hv) > 0) {
-    // One prep wave per chunk-head; valid offsets give at most T / C + N chunks.
-    const int64_t tc = (a.T + C - 1) / C;
-    PrefillArgs b = a;
-    b.prep_slots = int(tc + a.N - 1 < a.N * tc ? tc + a.N - 1 : a.N * tc);
-    const int64_t grid = (int64_t(b.prep_slots) * a.Hv + kPrepWaves - 1) / kPrepWaves;
-    hipLaunchKernelGGL(gdn_prefill_prep_kernel, dim3(unsigned(grid)), dim3(64 * kPrepWaves), 0, stream, b);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    if (F == 4) return launch_variant<Variant<2, 1, false, true>>(a, stream, done);
-    const int64_t chains = int64_t(a.N) * a.Hv;
-    const dim3 sgrid(unsigned((chains + 15) / 16 * 16 * kStateSlices)), sblock(512);
-    if (done != nullptr) {
-      hipExtLaunchKernelGGL(gdn_prefill_state_kernel, sgrid, sblock, 0, stream, nullptr, done, 0, a);
-    } else {
-      hipLaunchKernelGGL(gdn_prefill_state_kernel, sgrid, sblock, 0, stream, a);
-    }
-    return hipGetLastError();
-  }
+  if (a.tiles != nullptr && prefill_workspace_bytes(a.N, a.T, a.Hv) > 0)
+    return launch_two_kernels(a, stream, a.N * ((a.T + C - 1) / C), done);
   // Split chains use 16-row consumer waves (VT = 1), whose per-chunk chain is
   // shorter than a 32-row wave's.  Unsplit chains (F = 1) keep four 32-row waves:
   // eight 16-row waves and the four producers would exceed the register file.

@@ -166,12 +166,11 @@ int64_t gdn_static_device_bytes(void);
  * several workgroups (at most 64 (sequence, v-head) chains on 256 CUs) runs the
  * two-kernel path of gdn_prefill_with_workspace (each chunk prepared once) in a
  * scratch array the library holds on each device (GDN_PREFILL_DROPIN_SCRATCH_BYTES,
- * its own, not gdn_prefill_no_alloc's), when its chunk images fit:
- * gdn_prefill_workspace_size(num_seqs, total_tokens, Hv) bytes, 19,200 per 64-token
- * chunk and v-head of each sequence's ceil(total_tokens / 64) chunk slots, so with
- * one sequence and 32 v-heads up to 13,952 tokens (BASELINE's 4,096-token sequence
- * needs 37.5 MiB).  Larger batches run one kernel (one 16,384-token sequence: about
- * 8 % slower than two).  The results are the same bit for bit either way.  The library orders those launches on the device (each
+ * its own, not gdn_prefill_no_alloc's).  The chunk images take 19,200 bytes per 64-token
+ * chunk and v-head (one sequence with 32 v-heads: up to 13,952 tokens at a time;
+ * BASELINE's 4,096-token sequence needs 37.5 MiB); a batch that needs more runs in windows
+ * of its sequences, the state carried from one to the next.  The results are the same bit
+ * for bit either way.  The library orders those launches on the device (each
  * waits, on its stream, for an event that the previous one records as it
  * completes), so calls on any streams stay correct; on a stream that is being
  * captured into a graph such a call runs one kernel instead.

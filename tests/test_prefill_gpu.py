@@ -702,3 +702,26 @@ def test_prefill_dropin_long_sequence(gpu):
     assert_close(host(out), o_ref, OUT_RTOL, OUT_ATOL, "output")
     assert_close(host(ns), s_ref, STATE_RTOL, STATE_ATOL, "new_state")
     assert torch.equal(out, o2) and torch.equal(ns, s2)
+
+
+@pytest.mark.parametrize("lens,in_place", [
+    ([15001], True),           # one sequence, 32 chains: two windows
+    ([10500, 4700], False),    # 64 chains split 4 ways; one sequence ends in the first window
+])
+def test_prefill_dropin_windows(gpu, lens, in_place):
+    """Batches whose chunk images exceed the drop-in's scratch run in windows of the
+    sequences, the state carried from one to the next in new_state: against the oracle,
+    and bit for bit equal to gdn_prefill_with_workspace (one window)."""
+    say(f"prefill drop-in in windows, lens={lens} in_place={in_place}")
+    lib = _lib.load()
+    T, N = sum(lens), len(lens)
+    assert ((T + 63) // 64 + N - 1) * 32 * 19200 > _lib.GDN_PREFILL_DROPIN_SCRATCH_BYTES
+    assert lib.gdn_prefill_workspace_size(N, T, 32) > 0
+    p = workloads.prefill_inputs(lens, seed=64, gate="slow", state_scale=0.5)
+    o2, s2 = _prefill_capi(p, gpu, workspace=True)
+    o_ref, s_ref = oracle_prefill(p)
+    out, ns = run_prefill(p, gpu, in_place=in_place)
+    torch.cuda.synchronize()
+    assert torch.equal(out, o2) and torch.equal(ns, s2)
+    assert_close(host(out), o_ref, OUT_RTOL, OUT_ATOL, "output")
+    assert_close(host(ns), s_ref, STATE_RTOL, STATE_ATOL, "new_state")
