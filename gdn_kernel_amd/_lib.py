@@ -2,7 +2,8 @@
 
 The library is built in-tree by ``gdn_kernel_amd.build``.  There is no fallback
 implementation: if the shared object is missing or fails to load, every entry
-point raises.
+point raises.  The native module ``_native`` (csrc/gdn_torch.cpp), built beside it,
+is the short call path of the Python entry points.
 """
 from __future__ import annotations
 
@@ -59,6 +60,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_native = None
 
 
 class GDNError(RuntimeError):
@@ -85,6 +87,35 @@ def load() -> ctypes.CDLL:
         fn.restype = restype
     _lib = lib
     return lib
+
+
+class _NoNative:
+    """Where only the library was built: the Python code takes every call."""
+
+    @staticmethod
+    def decode(*args):
+        return None
+
+    decode_pooled = prefill = prefill_with_workspace = decode
+
+
+def native():
+    """Load (once) and return the native module, bound to the library's entry points."""
+    global _native
+    if _native is not None:
+        return _native
+    lib = load()
+    import torch
+    try:
+        from . import _native as mod
+    except ImportError:
+        _native = _NoNative
+        return _native
+    mod.bind(*(ctypes.cast(fn, c_void_p).value for fn in
+               (lib.gdn_decode, lib.gdn_decode_pooled, lib.gdn_prefill, lib.gdn_prefill_with_workspace)),
+             torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+    _native = mod
+    return mod
 
 
 def last_error() -> str:

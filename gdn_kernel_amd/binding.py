@@ -23,7 +23,9 @@ nothing), shapes, dtypes, devices and contiguity are validated and reported as
 ``ValueError``; device errors raise ``GDNError``.
 
 Tensors travel to the C ABI as raw device pointers; torch is used only for
-tensor metadata and the current HIP stream.
+tensor metadata and the current HIP stream.  Calls with plain tensors that need no
+message or device switch are checked and launched by the native module
+(csrc/gdn_torch.cpp); it returns None for all others, which run the code here.
 """
 from __future__ import annotations
 
@@ -105,6 +107,11 @@ def decode_kernel(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state
     q,k [B,1,H{q,k},128] bf16; v [B,1,Hv,128] bf16; state [B,Hv,128,128] fp32 or
     None; A_log,dt_bias [Hv] fp32; a,b [B,1,Hv] bf16; output [B,1,Hv,128] bf16;
     new_state [B,Hv,128,128] fp32 (may be ``state``)."""
+    rc = _lib.native().decode(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state)
+    if rc is not None:
+        if rc:
+            _lib.check(rc)
+        return
     dev = _device_of(q)
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be 4-D [B, 1, H, d]")
@@ -139,6 +146,11 @@ def decode_pooled_kernel(q, k, v, state_pool, A_log, a, dt_bias, b, scale, outpu
     an index outside [0, S) is a padding row (zero output, no slot touched).  Rows
     whose slot another row of the batch also names are skipped the same way, on the
     device, and counted (``decode_pool_conflicts``)."""
+    rc = _lib.native().decode_pooled(q, k, v, state_pool, A_log, a, dt_bias, b, scale, output, state_indices)
+    if rc is not None:
+        if rc:
+            _lib.check(rc)
+        return
     dev = _device_of(q)
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be 4-D [B, 1, H, d]")
@@ -223,6 +235,11 @@ def prefill_kernel(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, outp
     does: nothing is allocated, and calls on any streams give correct results (one long
     sequence runs two kernels in a scratch of the library, whose launches the library
     orders on the device)."""
+    rc = _lib.native().prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new_state)
+    if rc is not None:
+        if rc:
+            _lib.check(rc)
+        return
     dev, args = _prefill_args(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, output, new_state)
     args[12] = _scale(scale)
     lib = _lib.load()
@@ -248,6 +265,12 @@ def prefill_kernel_with_workspace(q, k, v, state, A_log, a, dt_bias, b, cu_seqle
     is a contiguous uint8 tensor of at least ``prefill_workspace_bytes(N, T, Hv)`` bytes
     on the same device (or None: ``prefill_kernel``); launches that may overlap must
     not share one."""
+    rc = _lib.native().prefill_with_workspace(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale,
+                                              output, new_state, workspace)
+    if rc is not None:
+        if rc:
+            _lib.check(rc)
+        return
     dev, args = _prefill_args(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, output, new_state)
     args[12] = _scale(scale)
     if workspace is not None:

@@ -1,4 +1,5 @@
-"""Build ``libgdn_kernel_amd.so`` (gfx950) in-tree with hipcc.
+"""Build ``libgdn_kernel_amd.so`` (gfx950) in-tree with hipcc, and the native module
+``_native`` of the Python entry points with the host compiler.
 
 Usage: ``python -m gdn_kernel_amd.build`` (or ``build()`` from Python).
 The shared library is written next to this file so that it travels with the
@@ -11,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -81,6 +83,35 @@ def build(verbose: bool = False, out: Path | None = None) -> Path:
     return out
 
 
+NATIVE_SOURCE = "gdn_torch.cpp"
+
+
+def native_path() -> Path:
+    return PKG_DIR / f"_native{sysconfig.get_config_var('EXT_SUFFIX')}"
+
+
+def build_native(verbose: bool = False) -> Path:
+    """Compile the native module of the Python entry points (host-only C++ over torch's
+    tensor headers; it takes the library's addresses at run time)."""
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    out = native_path()
+    tmp = out.with_name(out.name + ".tmp")
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "c++"
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           "-isystem", str(root / "include"), "-isystem", str(root / "include/torch/csrc/api/include"),
+           "-isystem", sysconfig.get_paths()["include"], str(CSRC / NATIVE_SOURCE),
+           "-L", str(root / "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-o", str(tmp)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("the native module failed to build:\n" + res.stdout + res.stderr)
+    os.replace(tmp, out)
+    return out
+
+
 # TVM-FFI exports (one `kernel` symbol per module, as the reference's two solutions):
 # host-only C++ over the C ABI, built when the tvm-ffi headers can be found.
 TVM_FFI_SHIMS = {"decode": "tvm_ffi/kernel.cpp", "prefill": "tvm_ffi/kernel_prefill.cpp"}
@@ -138,5 +169,6 @@ def build_tvm_ffi(verbose: bool = False, paths: dict | None = None) -> dict:
 if __name__ == "__main__":
     path = build(verbose="-v" in sys.argv)
     print(f"built {path}")
+    print(f"built {build_native(verbose='-v' in sys.argv)}")
     for op, p in build_tvm_ffi(verbose=True).items():
         print(f"built {p} (TVM-FFI `kernel`, {op})")
