@@ -88,12 +88,14 @@ constexpr int64_t kPrefillScratchBytes = int64_t(64) << 20;
 hipError_t prefill_scratch(void** ptr);
 
 // The drop-in gdn_prefill's launcher: launch_prefill, except that a batch of few
-// chains whose sequences average at least kDropinTwoKernelTokens tokens runs the
+// chains whose sequences average at least kDropinTwoKernelTokens tokens (split 8 ways:
+// kDropinTwoKernelTokens8) runs the
 // two-kernel path in a per-device scratch of the library (kPrefillDropinScratchBytes),
 // in windows of the sequences if its images do not fit, ordered between launches by an
 // event.
 constexpr int64_t kPrefillDropinScratchBytes = int64_t(128) << 20;
 constexpr int64_t kDropinTwoKernelTokens = 1024;
+constexpr int64_t kDropinTwoKernelTokens8 = 640;  // chains split 8 ways
 hipError_t launch_prefill_dropin(const PrefillArgs& args, hipStream_t stream);
 
 // gdn_prefill_no_alloc's launcher: the two-kernel path (for batches that take it) in

@@ -2971,24 +2971,43 @@ int64_t prefill_static_device_bytes() {
   return int64_t(sizeof(scratch)) + int64_t(sizeof(dropin_scratch)) + int64_t(sizeof(gdn_prefill_giveup_count));
 }
 
-// The drop-in gdn_prefill.  A batch of N sequences averaging at least
-// kDropinTwoKernelTokens tokens (T >= kDropinTwoKernelTokens N), whose chains the
-// launcher splits 4 or 8 ways, runs on the two-kernel path (each chunk prepared once)
-// in dropin_scratch, in windows if its images do not fit; everything else, and any launch
-// on a stream that is being captured into a graph, runs launch_prefill as is.  (The host sees N
-// and T, not the lengths; measured, one kernel against two, µs: [2048, 2048] 111.2 /
-// 99.2, [300, 4000] 189.4 / 150.2, [1000, 1100] 62.2 / 59.8, [900, 1200, 100, 3000]
-// at 16 v-heads 142.2 / 114.0, and below the threshold [600, 700] 42.5 / 42.4,
-// [512] x 4 at 16 v-heads 32.7 / 36.9.)  Launches on the scratch are ordered on the
-// device (launch_ordered), so calls on any streams stay correct, and calls on one
-// stream wait for nothing they would not wait for anyway.
 namespace {
 int split_factor(int64_t chains);
+
+// Whether the drop-in runs a batch on the two-kernel path.  The host sees N and T, not the
+// lengths, so the line is drawn by the average length, where equal lengths gain nothing yet
+// (ragged batches, which end with their longest chain, gain from there on).  One kernel
+// against two in the drop-in's scratch, us:
+//  * split 8 ways, from 640 tokens: one sequence at 32 v-heads 512 tokens 25.0 / 25.7, 640
+//    29.8 / 28.5, 768 34.5 / 31.2; two of 640 at 16 v-heads 30.4 / 29.8;
+//  * split 4 ways, from 1,024: [640, 640] 35.5 / 39.7, [900, 900] 49.1 / 48.9, [2048, 2048]
+//    111 / 86.0;
+//  * split 2 ways, from 1,024 where three eighths of the CUs or fewer have a chain: the
+//    state pass saves about a third of a chunk of the longest chain, the prep kernel adds
+//    10 us per 1,000 chunk-heads.  96 chains: [1024] x 3 63.6 / 61.5, [100, 3000, 900] 169.5 /
+//    127.6, [768] x 3 49.6 / 49.6; 128 chains: [1024] x 4 67.7 / 69.5, [2048] x 4 126.8 / 132.0
+//    (but [1000, 1500, 300, 1307] 93.0 / 86.6).
+// One or two sequences run in windows if their images do not fit the scratch; for more, as
+// offsets that overlap have to fit too (N ceil(T / C) images a v-head), windows would mostly
+// be empty (in twice the scratch, twelve sequences of 1,024 at 8 v-heads, two windows, the
+// second of them empty: 63.8 / 69.7).
+bool dropin_two_kernels(const PrefillArgs& a) {
+  const int64_t chains = int64_t(a.N) * a.Hv;
+  const int F = split_factor(chains);
+  if (F < 2 || (F == 2 && 8 * chains > 3 * int64_t(device_cus()))) return false;
+  if (a.T < (F == 8 ? kDropinTwoKernelTokens8 : kDropinTwoKernelTokens) * a.N) return false;
+  return a.N <= 2 || chains * ((a.T + C - 1) / C) * kTileImage * 16 <= kPrefillDropinScratchBytes;
 }
+}  // namespace
+
+// The drop-in gdn_prefill: batches of few chains with long sequences (dropin_two_kernels) on
+// the two-kernel path (each chunk prepared once) in dropin_scratch; everything else, and any
+// launch on a stream that is being captured into a graph, runs launch_prefill as is.
+// Launches on the scratch are ordered on the device (launch_ordered), so calls on any
+// streams stay correct, and calls on one stream wait for nothing they would not wait for
+// anyway.
 hipError_t launch_prefill_dropin(const PrefillArgs& a, hipStream_t stream) {
-  // (Room for at least one chunk a sequence: N Hv <= 64 images, see split_factor.)
-  if (a.T < kDropinTwoKernelTokens * a.N || split_factor(int64_t(a.N) * a.Hv) < 4 || a.spin_limit != 0 || a.ready_chunks != 0 ||
-      a.aborts != nullptr || a.tiles != nullptr)
+  if (!dropin_two_kernels(a) || a.spin_limit != 0 || a.ready_chunks != 0 || a.aborts != nullptr || a.tiles != nullptr)
     return launch_prefill(a, stream);
   hipError_t e = hipSuccess;
   if (stream_capturing(stream, &e)) return launch_prefill(a, stream);
@@ -3107,7 +3126,9 @@ hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const hipEvent_t last = i + 1 == windows ? done : nullptr;
-    if (split_factor(chains) == 4) {
+    if (split_factor(chains) == 2) {
+      e = launch_variant<Variant<4, 1, false, true>>(b, stream, last);
+    } else if (split_factor(chains) == 4) {
       e = launch_variant<Variant<2, 1, false, true>>(b, stream, last);
     } else {
       const dim3 sgrid(unsigned((chains + 15) / 16 * 16 * kStateSlices)), sblock(512);

@@ -161,15 +161,15 @@ int64_t gdn_static_device_bytes(void);
  *   output    [T,Hv,128] bf16
  *   new_state [N,Hv,128,128] fp32 final states; may alias state.
  * Nothing is allocated per call.  A batch whose sequences average at least
- * GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS (1,024) tokens (total_tokens >= 1,024
- * num_seqs) and whose chains the launcher splits over
- * several workgroups (at most 64 (sequence, v-head) chains on 256 CUs) runs the
- * two-kernel path of gdn_prefill_with_workspace (each chunk prepared once) in a
+ * GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS (1,024) tokens (total_tokens >= 1,024 num_seqs;
+ * 640 with at most 32 chains) and that has at most 96 (sequence, v-head) chains on 256 CUs
+ * runs the two-kernel path of gdn_prefill_with_workspace (each chunk prepared once) in a
  * scratch array the library holds on each device (GDN_PREFILL_DROPIN_SCRATCH_BYTES,
  * its own, not gdn_prefill_no_alloc's).  The chunk images take 19,200 bytes per 64-token
  * chunk and v-head (one sequence with 32 v-heads: up to 13,952 tokens at a time;
- * BASELINE's 4,096-token sequence needs 37.5 MiB); a batch that needs more runs in windows
- * of its sequences, the state carried from one to the next.  The results are the same bit
+ * BASELINE's 4,096-token sequence needs 37.5 MiB); one or two sequences that need more run
+ * in windows, the state carried from one to the next, and more sequences than fit with any
+ * offsets (num_seqs ceil(total_tokens / 64) chunks) run one kernel.  The results are the same bit
  * for bit either way.  The library orders those launches on the device (each
  * waits, on its stream, for an event that the previous one records as it
  * completes), so calls on any streams stay correct; on a stream that is being

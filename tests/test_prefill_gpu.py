@@ -725,3 +725,27 @@ def test_prefill_dropin_windows(gpu, lens, in_place):
     assert torch.equal(out, o2) and torch.equal(ns, s2)
     assert_close(host(out), o_ref, OUT_RTOL, OUT_ATOL, "output")
     assert_close(host(ns), s_ref, STATE_RTOL, STATE_ATOL, "new_state")
+
+
+@pytest.mark.parametrize("lens,heads,two_kernels", [
+    ([100, 2999, 900], Heads(16, 16, 32), True),     # 96 chains, split 2 ways
+    ([1100, 64, 2000, 1], Heads(12, 6, 24), False),  # the same, below the average length
+    ([1024, 1025, 1023], Heads(8, 16, 32), True),    # at the threshold, distinct head ratios
+    ([700, 630], Heads(8, 8, 16), True),             # split 8 ways, above 640 tokens
+    ([640], Heads(16, 16, 32), True),                # at it
+    ([639], Heads(16, 16, 32), False),
+])
+def test_prefill_dropin_rule_edges(gpu, lens, heads, two_kernels):
+    """Around the lines of the drop-in's choice between one kernel and two: bit for bit the
+    one kernel (launched through the testing entry point with its hooks off), and within
+    tolerance of the oracle.  (two_kernels: which side of the line; the results do not tell.)"""
+    say(f"prefill drop-in rule lens={lens} heads={heads} two_kernels={two_kernels}")
+    p = workloads.prefill_inputs(lens, heads, seed=65, gate="slow", state_scale=0.5)
+    o1, s1, aborts = _prefill_fault_injection(p, gpu, 0, 0)
+    o2, s2 = run_prefill(p, gpu)
+    torch.cuda.synchronize()
+    assert int(aborts.item()) == 0
+    assert torch.equal(o1, o2) and torch.equal(s1, s2)
+    o_ref, s_ref = oracle_prefill(p)
+    assert_close(host(o2), o_ref, OUT_RTOL, OUT_ATOL, "output")
+    assert_close(host(s2), s_ref, STATE_RTOL, STATE_ATOL, "new_state")
