@@ -53,36 +53,56 @@ __device__ __forceinline__ void store_state(float* p, float4 x) {
 
 // Whether a row other than `bi` of the batch's B slot indices names `slot`.  The
 // WAVES waves of a workgroup (all on the same batch row) each scan an interleaved
-// share of the indices, four 64-index blocks per pass, and OR their verdicts
-// through LDS.  Ends with a workgroup barrier when WAVES > 1.
+// share of the indices, kScanBlocks 64-index blocks a pass, and OR their verdicts
+// through LDS.
+//
+// load() issues the first pass's loads; the caller issues its state loads behind them
+// and then asks named_elsewhere(), so the indices come back (and the waves exchange
+// their verdicts) while the state is on its way: loads return in order, so in the
+// reverse order, or with the scan before the state's loads, one would wait out both
+// latencies one after the other.
+constexpr int kScanBlocks = 4;
 template <int WAVES>
-__device__ __forceinline__ bool slot_named_elsewhere(const int32_t* slots, int B, int bi, int slot, int lane,
-                                                     int wave) {
-  constexpr int STEP = 64 * WAVES;
-  bool hit = false;
-  for (int i0 = 64 * wave; i0 < B; i0 += 4 * STEP) {
-    int s[4];
+struct SlotScan {
+  static constexpr int STEP = 64 * WAVES;
+  int s[kScanBlocks];
+
+  __device__ __forceinline__ void load(const int32_t* slots, int B, int i0) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = i0 + u * STEP + lane;
-      s[u] = i < B ? slots[i] : -1;
+    for (int u = 0; u < kScanBlocks; ++u) s[u] = slots[min(i0 + u * STEP, B - 1)];
+  }
+  __device__ __forceinline__ bool hits(int B, int bi, int slot, int i0) const {
+    bool hit = false;
+#pragma unroll
+    for (int u = 0; u < kScanBlocks; ++u) {
+      const int i = i0 + u * STEP;
+      hit |= s[u] == slot && i < B && i != bi;
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) hit |= s[u] == slot && i0 + u * STEP + lane != bi;
+    return hit;
   }
-  const bool any = __builtin_amdgcn_ballot_w64(hit) != 0;
-  if constexpr (WAVES == 1) {
-    return any;
-  } else {
-    __shared__ int wave_hit[WAVES];
-    if (lane == 0) wave_hit[wave] = any;
-    __syncthreads();
-    int r = 0;
+  // Ends with a workgroup barrier when WAVES > 1.
+  __device__ __forceinline__ bool named_elsewhere(const int32_t* slots, int B, int bi, int slot, int lane, int wave) {
+    int i0 = 64 * wave + lane;
+    bool hit = hits(B, bi, slot, i0);
+    for (int done = kScanBlocks * STEP; done < B; done += kScanBlocks * STEP) {
+      i0 += kScanBlocks * STEP;
+      load(slots, B, i0);
+      hit |= hits(B, bi, slot, i0);
+    }
+    const bool any = __builtin_amdgcn_ballot_w64(hit) != 0;
+    if constexpr (WAVES == 1) {
+      return any;
+    } else {
+      __shared__ int wave_hit[WAVES];
+      if (lane == 0) wave_hit[wave] = any;
+      __syncthreads();
+      int r = 0;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) r |= wave_hit[w];
-    return r != 0;
+      for (int w = 0; w < WAVES; ++w) r |= wave_hit[w];
+      return r != 0;
+    }
   }
-}
+};
 
 // RPW rows per wave, WAVES waves per workgroup; a workgroup covers RPW*WAVES
 // rows of one head and 128 / (RPW*WAVES) workgroups cover one head.
@@ -110,37 +130,25 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_decode_kernel(DecodeArgs p) {
   uint16_t* outp = p.out + head * D + row0;
 
   int64_t shead = head;                             // index of the state block
+  int slot = 0;
+  SlotScan<WAVES> scan;
   if constexpr (POOLED) {
-    const int64_t slot = p.slots[bi];
+    slot = p.slots[bi];
     if (slot < 0 || slot >= p.pool_slots) {         // padding slot: zero output, no state
       if (lane < RPW) outp[lane] = 0;
       return;
     }
-    // A slot that two rows of the batch name would be updated by both at once: such
-    // rows are skipped like padding (zero output, slot untouched), decided before any
-    // state access, and the first wave of each counts its row once.
-    if (slot_named_elsewhere<WAVES>(p.slots, p.B, bi, int(slot), lane, wave)) {
-      if (lane < RPW) outp[lane] = 0;
-      if (h == 0 && row0 == 0 && lane == 0)
-        __hip_atomic_fetch_add(&gdn_decode_pool_conflict_count, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return;
-    }
-    shead = slot * p.Hv + h;
+    scan.load(p.slots, p.B, 64 * wave + lane);
+    __builtin_amdgcn_sched_barrier(0);
+    shead = int64_t(slot) * p.Hv + h;
   }
 
-  // Gate and beta (every lane computes the same scalars).
-  const float g = expf(log_gate(p.A_log[h], bf16_to_f32(p.a[head]), p.dt_bias[h]));
-  const float beta = sigmoidf_(bf16_to_f32(p.b[head]));
-
-  // This lane's 4 columns of q and k.
   const int hq = h / (p.Hv / p.Hq);
   const int hk = h / (p.Hv / p.Hk);
+  const uint16_t a16 = p.a[head], b16 = p.b[head];
   const uint2 qw = *reinterpret_cast<const uint2*>(p.q + (int64_t(bi) * p.Hq + hq) * D + col);
   const uint2 kw = *reinterpret_cast<const uint2*>(p.k + (int64_t(bi) * p.Hk + hk) * D + col);
-  const float q0 = __uint_as_float(qw.x << 16), q1 = __uint_as_float(qw.x & 0xffff0000u);
-  const float q2 = __uint_as_float(qw.y << 16), q3 = __uint_as_float(qw.y & 0xffff0000u);
-  const float k0 = __uint_as_float(kw.x << 16), k1 = __uint_as_float(kw.x & 0xffff0000u);
-  const float k2 = __uint_as_float(kw.y << 16), k3 = __uint_as_float(kw.y & 0xffff0000u);
+  const uint16_t v16 = p.v[head * D + row0 + (RPW < 64 ? lane & (RPW - 1) : lane)];
 
   // Issue every state load of this wave before any arithmetic.
   const int64_t sbase = (shead * D + row0 + half) * D + col;
@@ -153,7 +161,30 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_decode_kernel(DecodeArgs p) {
     for (int j = 0; j < NL; ++j) s[j] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 
-  const float vmine = lane < RPW ? bf16_to_f32(p.v[head * D + row0 + lane]) : 0.0f;
+  if constexpr (POOLED) {
+    // A slot that two rows of the batch name would be updated by both at once: such
+    // rows are skipped like padding (zero output, slot untouched), decided before any
+    // state is written, and the first wave of each counts its row once.
+    __builtin_amdgcn_sched_barrier(0);
+    if (scan.named_elsewhere(p.slots, p.B, bi, slot, lane, wave)) {
+      if (lane < RPW) outp[lane] = 0;
+      if (h == 0 && row0 == 0 && lane == 0)
+        __hip_atomic_fetch_add(&gdn_decode_pool_conflict_count, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+  }
+
+  // Gate and beta (every lane computes the same scalars).
+  const float g = expf(log_gate(p.A_log[h], bf16_to_f32(a16), p.dt_bias[h]));
+  const float beta = sigmoidf_(bf16_to_f32(b16));
+
+  // This lane's 4 columns of q and k.
+  const float q0 = __uint_as_float(qw.x << 16), q1 = __uint_as_float(qw.x & 0xffff0000u);
+  const float q2 = __uint_as_float(qw.y << 16), q3 = __uint_as_float(qw.y & 0xffff0000u);
+  const float k0 = __uint_as_float(kw.x << 16), k1 = __uint_as_float(kw.x & 0xffff0000u);
+  const float k2 = __uint_as_float(kw.y << 16), k3 = __uint_as_float(kw.y & 0xffff0000u);
+
+  const float vmine = bf16_to_f32(v16);
   const float qdotk = sum32(q0 * k0 + q1 * k1 + q2 * k2 + q3 * k3);
 
   float myout = 0.0f;
