@@ -60,7 +60,8 @@ __device__ __forceinline__ void store_state(float* p, float4 x) {
 // and then asks named_elsewhere(), so the indices come back (and the waves exchange
 // their verdicts) while the state is on its way: loads return in order, so in the
 // reverse order, or with the scan before the state's loads, one would wait out both
-// latencies one after the other.
+// latencies one after the other (16 q / 16 k / 32 v heads, B = 512 of 1,024 slots: 374 us
+// with the scan first, 361 so; B = 24 of 64 slots 16.4, 16.0).
 constexpr int kScanBlocks = 4;
 template <int WAVES>
 struct SlotScan {

@@ -202,6 +202,34 @@ def test_decode_pooled_duplicate_slots(gpu, heads, B, slots):
     assert_close(host(pool), pool_ref, STATE_RTOL, STATE_ATOL, "pool")
 
 
+@pytest.mark.conflicts_expected
+@pytest.mark.parametrize("B", [2, 64, 65, 127, 128, 255, 257, 1024, 1025])
+def test_decode_pooled_scan_edges(gpu, B):
+    """The index scan at the ends of its blocks and passes (one-wave workgroups below 128
+    rows): the last row is not its own conflict where lanes past the batch read its index
+    again, and is one when the first row names its slot."""
+    say(f"decode pooled scan edges B={B}")
+    slots = B + 3
+    w = workloads.decode_inputs(B, Heads(1, 1, 1), seed=50 + B, gate="slow", pool_slots=slots, state_scale=1.0)
+    d = {k: (v.to(gpu) if isinstance(v, torch.Tensor) else v) for k, v in w.items()}
+    for shared in (False, True):
+        idx = w["state_indices"].clone()
+        if shared:
+            idx[B - 1] = idx[0]
+        conflict = O.pool_conflicts(idx.numpy(), slots)
+        assert int(conflict.sum()) == (2 if shared else 0)
+        o_ref, pool_ref = O.decode_pooled(*[to_numpy(w[k]) for k in ("q", "k", "v", "state")], idx.numpy(),
+                                          *[to_numpy(w[k]) for k in ("A_log", "a", "dt_bias", "b")], w["scale"])
+        pool, out = d["state"].clone(), torch.full_like(d["v"], float("nan"))
+        binding.decode_pool_conflicts(reset=True)
+        binding.decode_pooled_kernel(d["q"], d["k"], d["v"], pool, d["A_log"], d["a"], d["dt_bias"], d["b"],
+                                     d["scale"], out, idx.to(gpu))
+        assert binding.decode_pool_conflicts(reset=True) == int(conflict.sum())
+        assert not host(out)[conflict].any()
+        assert_close(host(out), o_ref, OUT_RTOL, OUT_ATOL, "output")
+        assert_close(host(pool), pool_ref, STATE_RTOL, STATE_ATOL, "pool")
+
+
 @pytest.mark.parametrize("B", [1, 8])
 def test_decode_edge_gates(gpu, B):
     """The gate prologue's edge branches against the oracle: softplus arguments above 20,
