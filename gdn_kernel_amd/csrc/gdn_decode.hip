@@ -120,11 +120,12 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_decode_kernel(DecodeArgs p) {
   const int half = lane >> 5;
   const int col = (lane & 31) * 4;
 
-  int blk = blockIdx.x;
-  const int rblk = blk % WG_PER_HEAD;
-  blk /= WG_PER_HEAD;
-  const int h = blk % p.Hv;
-  const int bi = blk / p.Hv;
+  // Unsigned, and by ratios formed on the host: a wave starts with these divisions, and its
+  // first state load waits for them (131 instructions before it instead of 196; plain
+  // B = 64 42.76 -> 42.47 us, pooled B = 24 15.80 -> 15.64).
+  const uint32_t rblk = blockIdx.x % WG_PER_HEAD, blk = blockIdx.x / WG_PER_HEAD;
+  const int bi = blk / uint32_t(p.Hv);
+  const int h = blk - uint32_t(bi) * uint32_t(p.Hv);
   const int row0 = rblk * ROWS_PER_WG + wave * RPW;
 
   const int64_t head = int64_t(bi) * p.Hv + h;     // index of (b, h) in v/a/b/out
@@ -144,8 +145,8 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_decode_kernel(DecodeArgs p) {
     shead = int64_t(slot) * p.Hv + h;
   }
 
-  const int hq = h / (p.Hv / p.Hq);
-  const int hk = h / (p.Hv / p.Hk);
+  const int hq = uint32_t(h) / uint32_t(p.q_group);
+  const int hk = uint32_t(h) / uint32_t(p.k_group);
   const uint16_t a16 = p.a[head], b16 = p.b[head];
   const uint2 qw = *reinterpret_cast<const uint2*>(p.q + (int64_t(bi) * p.Hq + hq) * D + col);
   const uint2 kw = *reinterpret_cast<const uint2*>(p.k + (int64_t(bi) * p.Hk + hk) * D + col);
@@ -220,7 +221,10 @@ namespace {
 static_assert(kDecodeVariants == 16, "the variant table has 16 entries");
 
 template <int RPW, int WAVES, bool NT>
-hipError_t launch_variant(const DecodeArgs& a, hipStream_t stream) {
+hipError_t launch_variant(const DecodeArgs& args, hipStream_t stream) {
+  DecodeArgs a = args;
+  a.q_group = a.Hv / a.Hq;
+  a.k_group = a.Hv / a.Hk;
   const int64_t heads = int64_t(a.B) * a.Hv;
   const int64_t grid = heads * (kHeadDim / (RPW * WAVES));
   const dim3 block(64 * WAVES);

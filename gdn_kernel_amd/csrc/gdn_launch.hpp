@@ -22,6 +22,7 @@ struct DecodeArgs {
   uint16_t* out;            // [B, Hv, 128] bf16
   float scale;
   int B, Hq, Hk, Hv;
+  int q_group, k_group;     // v-heads a q-head, a k-head; set by the launcher
 };
 
 struct PrefillArgs {
