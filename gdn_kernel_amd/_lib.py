@@ -23,6 +23,7 @@ GDN_MAX_HEADS = 65536
 GDN_PREFILL_NO_ALLOC_SCRATCH_BYTES = 64 << 20
 GDN_PREFILL_DROPIN_SCRATCH_BYTES = 128 << 20
 GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS = 1024
+GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS_8 = 640
 
 # Exported symbols and their argument types (must match include/gdn_kernel_amd.h and
 # include/gdn_kernel_amd_testing.h).
@@ -57,6 +58,8 @@ SIGNATURES = {
                                         c_int64] + _HEADS + [c_int32, _P], c_int),
     "gdn_prefill_fault_injection": ([_P] * 8 + [_P, c_int32, c_int64, c_int64, c_double, _P, _P]
                                     + _HEADS + [c_int32, c_int32, _P, _P], c_int),
+    "gdn_prefill_dropin_windows": ([c_int64, c_int64, c_int32, ctypes.POINTER(c_int32)], c_int64),
+    "gdn_prefill_dropin_held": ([ctypes.POINTER(c_int32), _P], c_int),
 }
 
 _lib = None

@@ -41,6 +41,8 @@ static_assert(GDN_PREFILL_DROPIN_SCRATCH_BYTES == gdn::kPrefillDropinScratchByte
               "the header's drop-in scratch size must match the library's");
 static_assert(GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS == gdn::kDropinTwoKernelTokens,
               "the header's drop-in two-kernel threshold must match the library's");
+static_assert(GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS_8 == gdn::kDropinTwoKernelTokens8,
+              "the header's drop-in two-kernel threshold (split 8 ways) must match the library's");
 
 int check_heads(int32_t hq, int32_t hk, int32_t hv, int32_t dk, int32_t dv) {
   if (hq <= 0 || hk <= 0 || hv <= 0)
@@ -372,6 +374,22 @@ int gdn_prefill_giveups(uint64_t* count, int32_t reset) {
 int gdn_decode_pool_conflicts(uint64_t* count, int32_t reset) {
   if (!count) return fail(GDN_ERR_INVALID_ARGUMENT, "count must not be null");
   return device_status(gdn::decode_pool_conflicts(count, reset != 0), "gdn_decode_pool_conflicts");
+}
+
+int64_t gdn_prefill_dropin_windows(int64_t num_seqs, int64_t total_tokens, int32_t num_v_heads, int32_t* yields) {
+  gdn::PrefillRoute r = {0, false};
+  if (num_seqs > 0 && num_seqs <= INT32_MAX && num_v_heads > 0)
+    r = gdn::dropin_route(int(num_seqs), total_tokens, num_v_heads);
+  if (yields) *yields = r.yields;
+  return r.windows;
+}
+
+int gdn_prefill_dropin_held(int32_t* held, void* stream) {
+  if (!held) return fail(GDN_ERR_INVALID_ARGUMENT, "held must not be null");
+  bool h = false;
+  const hipError_t e = gdn::dropin_held(static_cast<hipStream_t>(stream), &h);
+  *held = h;
+  return device_status(e, "gdn_prefill_dropin_held");
 }
 
 int gdn_decode_num_variants(void) { return gdn::kDecodeVariants; }

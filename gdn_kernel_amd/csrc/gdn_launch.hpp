@@ -93,11 +93,21 @@ hipError_t prefill_scratch(void** ptr);
 // kDropinTwoKernelTokens8) runs the
 // two-kernel path in a per-device scratch of the library (kPrefillDropinScratchBytes),
 // in windows of the sequences if its images do not fit, ordered between launches by an
-// event.
+// event (dropin_route has the rule).
 constexpr int64_t kPrefillDropinScratchBytes = int64_t(128) << 20;
 constexpr int64_t kDropinTwoKernelTokens = 1024;
 constexpr int64_t kDropinTwoKernelTokens8 = 640;  // chains split 8 ways
 hipError_t launch_prefill_dropin(const PrefillArgs& args, hipStream_t stream);
+
+// The drop-in's choice for a batch: the windows of the two-kernel path it runs in (0: one
+// kernel), and whether it yields (runs one kernel) while another stream's launch holds the
+// scratch; and whether one does now, for a launch on `stream`.
+struct PrefillRoute {
+  int64_t windows;
+  bool yields;
+};
+PrefillRoute dropin_route(int N, int64_t T, int Hv);
+hipError_t dropin_held(hipStream_t stream, bool* held);
 
 // gdn_prefill_no_alloc's launcher: the two-kernel path (for batches that take it) in
 // the kPrefillScratchBytes array; eager launches are ordered between each other by an

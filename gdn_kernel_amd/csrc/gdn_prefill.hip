@@ -66,6 +66,7 @@
 
 #include <atomic>
 #include <mutex>
+#include <thread>
 #include <type_traits>
 
 #include "gdn_common.hpp"
@@ -2891,32 +2892,65 @@ constexpr int kMaxDevices = 64;
 // the device current: in host code the array's name is a host-side stand-in), the
 // event that follows the last launch using it, and the lock that orders the
 // check-launch-record sequence between host threads.  Created on first use and
-// kept until the process ends, like the array itself.
+// kept until the process ends, like the array itself.  The stream (and thread, for the
+// per-thread default stream) of the last launch only decides whether a batch that yields
+// takes the array: what keeps launches apart is the event.
 struct OrderedScratch {
   std::mutex lock;
   void* addr = nullptr;
   hipEvent_t done = nullptr;
   bool used = false;
+  hipStream_t stream = nullptr;
+  std::thread::id thread;
 };
 OrderedScratch g_dropin[kMaxDevices];
 OrderedScratch g_no_alloc[kMaxDevices];
+
+hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t slots, hipEvent_t done);
+
+// The array's entry for the current device.
+hipError_t ordered_scratch(OrderedScratch* table, OrderedScratch** entry) {
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
+  *entry = table + dev;
+  return hipSuccess;
+}
+
+// Whether another stream's launch holds the array (its lock held by the caller): a launch
+// on `stream` would wait for it.
+bool held_by_another(const OrderedScratch& d, hipStream_t stream) {
+  if (!d.used) return false;
+  if (d.stream == stream && (stream != hipStreamPerThread || d.thread == std::this_thread::get_id())) return false;
+  // (An event query is not allowed while any thread captures a graph in the global mode,
+  // unless the querying thread has relaxed its own.)
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return true;
+  const hipError_t q = hipEventQuery(d.done);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (q != hipSuccess) (void)hipGetLastError();  // not ready
+  return q != hipSuccess;
+}
 
 // Launches the two-kernel path of `a` with its chunk images in the scratch array
 // `symbol`, ordered after the previous launch that used the array on this device:
 // the stream waits for that launch's event, and the state pass records the event
 // again as it completes.  If the launch fails after the prep kernel was enqueued,
 // the event is recorded behind it all the same, so the next launch still waits for
-// the orphaned kernel.
-hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t slots, hipEvent_t done);
-
+// the orphaned kernel.  With `yields`, runs launch_prefill instead if the array is held
+// by another stream's launch.
 hipError_t launch_ordered(const PrefillArgs& a, hipStream_t stream, OrderedScratch* table, const void* symbol,
-                          int64_t bytes) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
+                          int64_t bytes, bool yields) {
+  OrderedScratch* entry = nullptr;
+  hipError_t e = ordered_scratch(table, &entry);
   if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-  OrderedScratch& d = table[dev];
-  std::lock_guard<std::mutex> guard(d.lock);
+  OrderedScratch& d = *entry;
+  std::unique_lock<std::mutex> guard(d.lock);
+  if (yields && held_by_another(d, stream)) {
+    guard.unlock();
+    return launch_prefill(a, stream);
+  }
   if (d.addr == nullptr) {
     e = hipGetSymbolAddress(&d.addr, symbol);
     if (e != hipSuccess) return e;
@@ -2938,6 +2972,8 @@ hipError_t launch_ordered(const PrefillArgs& a, hipStream_t stream, OrderedScrat
     (void)hipEventRecord(d.done, stream);
   }
   d.used = true;
+  d.stream = stream;
+  d.thread = std::this_thread::get_id();
   return e;
 }
 
@@ -2974,8 +3010,25 @@ int64_t prefill_static_device_bytes() {
 namespace {
 int split_factor(int64_t chains);
 
-// Whether the drop-in runs a batch on the two-kernel path.  The host sees N and T, not the
-// lengths, so the line is drawn by the average length, where equal lengths gain nothing yet
+// Windows of the two-kernel path with room for `slots` chunk images a v-head (at least N):
+// their number and the chunks of each sequence that one covers.  If the chunks that any
+// offsets can give do not fit (one or two sequences cannot overlap: at most ceil(T / C) + N
+// - 1; more, if malformed, can: N ceil(T / C)), the batch runs in windows of equally many
+// chunks of every sequence.
+struct Windows {
+  int64_t count, chunks;
+};
+Windows plan_windows(int64_t N, int64_t T, int64_t slots) {
+  const int64_t tc = (T + C - 1) / C;
+  const int64_t most = N <= 2 ? tc + N - 1 : N * tc;  // chunks any offsets can give
+  const int64_t fit = most <= slots ? tc : slots / N;  // chunks of a sequence a window
+  const int64_t count = (tc + fit - 1) / fit;
+  return Windows{count, (tc + count - 1) / count};
+}
+}  // namespace
+
+// How the drop-in runs a batch.  The host sees N and T, not the lengths, so the line between
+// one kernel and two is drawn by the average length, where equal lengths gain nothing yet
 // (ragged batches, which end with their longest chain, gain from there on).  One kernel
 // against two in the drop-in's scratch, us:
 //  * split 8 ways, from 640 tokens: one sequence at 32 v-heads 512 tokens 25.0 / 25.7, 640
@@ -2987,32 +3040,61 @@ int split_factor(int64_t chains);
 //    10 us per 1,000 chunk-heads.  96 chains: [1024] x 3 63.6 / 61.5, [100, 3000, 900] 169.5 /
 //    127.6, [768] x 3 49.6 / 49.6; 128 chains: [1024] x 4 67.7 / 69.5, [2048] x 4 126.8 / 132.0
 //    (but [1000, 1500, 300, 1307] 93.0 / 86.6).
+//
+// Launches in the scratch run one after another, whatever their streams.  Below 1,024 tokens,
+// and split 2 ways, that costs calls on several streams more than two kernels give them, so
+// those batches yield: one kernel while another stream's launch holds the scratch.  A call
+// on each of several streams, us, one kernel / two kernels in turn / yielding: [700] at 16
+// v-heads on two streams 39.5 / 72 / 34, at 32 62 / 77 / 61, at 8 on four 79 / 141 / 80;
+// [1024] x 3 at 32 on two 94.5 / 125 / 89; [4096, 4096] at 48 356 / 431 / 348.
+//
 // One or two sequences run in windows if their images do not fit the scratch; for more, as
 // offsets that overlap have to fit too (N ceil(T / C) images a v-head), windows would mostly
 // be empty (in twice the scratch, twelve sequences of 1,024 at 8 v-heads, two windows, the
-// second of them empty: 63.8 / 69.7).
-bool dropin_two_kernels(const PrefillArgs& a) {
-  const int64_t chains = int64_t(a.N) * a.Hv;
+// second of them empty: 63.8 / 69.7).  Windows hold the scratch for long, so they are for
+// batches that leave other streams little room anyway, with a workgroup on three quarters of
+// the CUs: a call on each of two streams, one kernel / windows, [16384] at 32 v-heads 1,196 /
+// 845, at 24 v-heads 20,000 tokens 1,464 / 988; but at 16 v-heads 30,000 tokens 1,099 /
+// 1,353, at 8 60,000 2,204 / 2,549, and split 2 ways [8192, 8192] at 48 706 / 903.
+PrefillRoute dropin_route(int N, int64_t T, int Hv) {
+  const PrefillRoute one_kernel = {0, false};
+  if (N <= 0 || T <= 0) return one_kernel;
+  const int64_t chains = int64_t(N) * Hv, cus = device_cus();
   const int F = split_factor(chains);
-  if (F < 2 || (F == 2 && 8 * chains > 3 * int64_t(device_cus()))) return false;
-  if (a.T < (F == 8 ? kDropinTwoKernelTokens8 : kDropinTwoKernelTokens) * a.N) return false;
-  return a.N <= 2 || chains * ((a.T + C - 1) / C) * kTileImage * 16 <= kPrefillDropinScratchBytes;
+  if (F < 2 || (F == 2 && 8 * chains > 3 * cus)) return one_kernel;
+  if (T < (F == 8 ? kDropinTwoKernelTokens8 : kDropinTwoKernelTokens) * N) return one_kernel;
+  PrefillRoute r = {1, F == 2 || T < kDropinTwoKernelTokens * N};
+  if (chains * ((T + C - 1) / C) * kTileImage * 16 > kPrefillDropinScratchBytes) {
+    if (N > 2) return one_kernel;
+    r.windows = plan_windows(N, T, kPrefillDropinScratchBytes / (int64_t(Hv) * kTileImage * 16)).count;
+    if (F == 2 ? r.windows > 1 : 4 * chains * F < 3 * cus) return one_kernel;
+  }
+  return r;
 }
-}  // namespace
 
-// The drop-in gdn_prefill: batches of few chains with long sequences (dropin_two_kernels) on
-// the two-kernel path (each chunk prepared once) in dropin_scratch; everything else, and any
+// The drop-in gdn_prefill: batches of few chains with long sequences (dropin_route) on the
+// two-kernel path (each chunk prepared once) in dropin_scratch; everything else, and any
 // launch on a stream that is being captured into a graph, runs launch_prefill as is.
 // Launches on the scratch are ordered on the device (launch_ordered), so calls on any
 // streams stay correct, and calls on one stream wait for nothing they would not wait for
 // anyway.
 hipError_t launch_prefill_dropin(const PrefillArgs& a, hipStream_t stream) {
-  if (!dropin_two_kernels(a) || a.spin_limit != 0 || a.ready_chunks != 0 || a.aborts != nullptr || a.tiles != nullptr)
+  const PrefillRoute r = dropin_route(a.N, a.T, a.Hv);
+  if (r.windows == 0 || a.spin_limit != 0 || a.ready_chunks != 0 || a.aborts != nullptr || a.tiles != nullptr)
     return launch_prefill(a, stream);
   hipError_t e = hipSuccess;
   if (stream_capturing(stream, &e)) return launch_prefill(a, stream);
   if (e != hipSuccess) return e;
-  return launch_ordered(a, stream, g_dropin, HIP_SYMBOL(dropin_scratch), kPrefillDropinScratchBytes);
+  return launch_ordered(a, stream, g_dropin, HIP_SYMBOL(dropin_scratch), kPrefillDropinScratchBytes, r.yields);
+}
+
+hipError_t dropin_held(hipStream_t stream, bool* held) {
+  OrderedScratch* d = nullptr;
+  const hipError_t e = ordered_scratch(g_dropin, &d);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> guard(d->lock);
+  *held = held_by_another(*d, stream);
+  return hipSuccess;
 }
 
 // gdn_prefill_no_alloc: the two-kernel path in `scratch` for batches that take it.
@@ -3032,7 +3114,7 @@ hipError_t launch_prefill_no_alloc(const PrefillArgs& a, hipStream_t stream) {
     return launch_prefill(b, stream);
   }
   if (e != hipSuccess) return e;
-  return launch_ordered(a, stream, g_no_alloc, HIP_SYMBOL(scratch), kPrefillScratchBytes);
+  return launch_ordered(a, stream, g_no_alloc, HIP_SYMBOL(scratch), kPrefillScratchBytes, false);
 }
 
 // Reads (and with `reset` clears) this device's give-up count, after
@@ -3099,19 +3181,15 @@ int64_t prefill_workspace_bytes(int N, int64_t T, int Hv) {
 }
 
 namespace {
-// The two-kernel path with room for `slots` chunk images a v-head (at least N).  If the
-// chunks that any offsets can give do not fit (one or two sequences cannot overlap: at most
-// ceil(T / C) + N - 1; more, if malformed, can: N ceil(T / C)), the batch runs in windows of
-// equally many chunks of every sequence, each a prep kernel and a state pass that takes the
-// state up where the window before left it, in new_state: the same operations in the same
-// order.  A window costs about 8 us (the launches, and both kernels filling and draining
-// the chip); one 16,384-token sequence at 32 v-heads takes 412 us in two windows, 598 in one
-// kernel.
+// The two-kernel path with room for `slots` chunk images a v-head (at least N), in
+// plan_windows' windows, each a prep kernel and a state pass that takes the state up where
+// the window before left it, in new_state: the same operations in the same order.  A window
+// costs about 8 us (the launches, and both kernels filling and draining the chip); one
+// 16,384-token sequence at 32 v-heads takes 412 us in two windows, 598 in one kernel.
 hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t slots, hipEvent_t done) {
   const int64_t tc = (a.T + C - 1) / C;
-  const int64_t most = a.N <= 2 ? tc + a.N - 1 : a.N * tc;  // chunks any offsets can give
-  const int64_t fit = most <= slots ? tc : slots / a.N;     // chunks of a sequence a window
-  const int64_t windows = (tc + fit - 1) / fit, w = (tc + windows - 1) / windows;
+  const Windows plan = plan_windows(a.N, a.T, slots);
+  const int64_t windows = plan.count, w = plan.chunks;
   // Valid offsets give at most T / C + N chunks.
   PrefillArgs b = a;
   b.prep_slots = int(tc + a.N - 1 < a.N * w ? tc + a.N - 1 : a.N * w);

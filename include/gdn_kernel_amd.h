@@ -25,7 +25,7 @@
  *     device and for their own scratch array, the array's address, a mutex and one
  *     event (created on first use and kept) that orders their two-kernel launches
  *     on that device (each such launch waits, on its stream, for the event the
- *     previous one recorded).  The two device counters (prefill hand-off give-ups,
+ *     previous one recorded), and gdn_prefill the stream of its last such launch.  The two device counters (prefill hand-off give-ups,
  *     pooled-decode slot conflicts) persist between calls until their query resets
  *     them.  The decode entry points keep no other state.
  *   - Thread safety: every entry point may be called from any host thread; the
@@ -162,21 +162,25 @@ int64_t gdn_static_device_bytes(void);
  *   new_state [N,Hv,128,128] fp32 final states; may alias state.
  * Nothing is allocated per call.  A batch whose sequences average at least
  * GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS (1,024) tokens (total_tokens >= 1,024 num_seqs;
- * 640 with at most 32 chains) and that has at most 96 (sequence, v-head) chains on 256 CUs
- * runs the two-kernel path of gdn_prefill_with_workspace (each chunk prepared once) in a
+ * GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS_8, 640, with at most 32 chains) and that has at most
+ * 96 (sequence, v-head) chains on 256 CUs runs the two-kernel path of gdn_prefill_with_workspace (each chunk prepared once) in a
  * scratch array the library holds on each device (GDN_PREFILL_DROPIN_SCRATCH_BYTES,
  * its own, not gdn_prefill_no_alloc's).  The chunk images take 19,200 bytes per 64-token
  * chunk and v-head (one sequence with 32 v-heads: up to 13,952 tokens at a time;
- * BASELINE's 4,096-token sequence needs 37.5 MiB); one or two sequences that need more run
- * in windows, the state carried from one to the next, and more sequences than fit with any
- * offsets (num_seqs ceil(total_tokens / 64) chunks) run one kernel.  The results are the same bit
- * for bit either way.  The library orders those launches on the device (each
+ * BASELINE's 4,096-token sequence needs 37.5 MiB); one or two sequences that need more and
+ * have 24 to 32 or 48 to 64 chains (a workgroup on three quarters of the CUs) run in windows,
+ * the state carried from one to the next, and others that do not fit (more sequences: with
+ * any offsets, num_seqs ceil(total_tokens / 64) chunks) run one kernel.  The results are the
+ * same bit for bit either way.  The library orders those launches on the device (each
  * waits, on its stream, for an event that the previous one records as it
- * completes), so calls on any streams stay correct; on a stream that is being
- * captured into a graph such a call runs one kernel instead.
+ * completes), so calls on any streams stay correct.  A batch of more than 64 chains, or of
+ * less than 1,024 tokens a sequence, does not wait for another stream: while a launch of
+ * another stream holds the scratch it runs one kernel, and so does any batch on a stream
+ * that is being captured into a graph.
  */
 #define GDN_PREFILL_DROPIN_SCRATCH_BYTES (128LL << 20)
 #define GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS 1024
+#define GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS_8 640
 
 int gdn_prefill(const gdn_bf16* q, const gdn_bf16* k, const gdn_bf16* v,
                 const float* state, const float* A_log, const gdn_bf16* a,

@@ -40,6 +40,17 @@ int gdn_prefill_fault_injection(const gdn_bf16* q, const gdn_bf16* k, const gdn_
                                 int32_t ready_chunks, uint32_t* aborts, void* stream);
 
 /*
+ * How gdn_prefill runs a batch outside graph capture: the number of windows of the
+ * two-kernel path (0: one kernel).  *yields (if not null) is 1 for a batch that runs one
+ * kernel all the same while a launch of another stream holds the library's scratch;
+ * gdn_prefill_dropin_held stores in *held whether one does now, for a call on `stream`.
+ * Neither launches anything.
+ */
+int64_t gdn_prefill_dropin_windows(int64_t num_seqs, int64_t total_tokens, int32_t num_v_heads,
+                                   int32_t* yields);
+int gdn_prefill_dropin_held(int32_t* held, void* stream);
+
+/*
  * Decode with an explicit launch shape instead of the batch-size heuristic, so that
  * tests can check every compiled shape and tuning runs can time them.  Arguments as
  * gdn_decode / gdn_decode_pooled plus `variant` in [0, gdn_decode_num_variants()):

@@ -119,7 +119,7 @@ def test_header_constants_match_the_python_binding():
     defs = dict(re.findall(r"^#define (GDN_[A-Z0-9_]+) \(?([0-9LL <]+?)\)?\s*(?:/\*.*)?$", text, re.M))
     assert {"GDN_OK", "GDN_ERR_UNSUPPORTED", "GDN_INDEX_INT64", "GDN_MAX_HEADS",
             "GDN_PREFILL_NO_ALLOC_SCRATCH_BYTES", "GDN_PREFILL_DROPIN_SCRATCH_BYTES",
-            "GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS"} <= set(defs)
+            "GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS", "GDN_PREFILL_DROPIN_TWO_KERNEL_TOKENS_8"} <= set(defs)
     for name, value in defs.items():
         parts = [int(x.strip().rstrip("L")) for x in value.split("<<")]
         expected = parts[0] << parts[1] if len(parts) == 2 else parts[0]
@@ -194,6 +194,28 @@ def test_prefill_workspace_size(lib):
     for n, t, hv in ((0, 100, 8), (1, 0, 8), (1, 100, 0), (-1, 100, 8), (1, -5, 8)):
         assert lib.gdn_prefill_workspace_size(n, t, hv) == 0
     assert lib.gdn_prefill_workspace_size(1, 1 << 24, 32) == 0                   # above the 2 GiB cap
+
+
+@pytest.mark.parametrize("N,T,hv,windows,yields", [
+    (1, 639, 32, 0, 0), (1, 640, 32, 1, 1), (2, 1279, 16, 0, 0), (2, 1280, 16, 1, 1),  # split 8 ways: 640 a sequence
+    (1, 1023, 8, 1, 1), (1, 1024, 8, 1, 0),                                 # from 1,024 on ordered
+    (2, 2047, 32, 0, 0), (2, 2048, 32, 1, 0), (1, 1024, 33, 1, 0),          # split 4 ways: 1,024
+    (3, 3071, 32, 0, 0), (3, 3072, 32, 1, 1), (1, 1024, 96, 1, 1),          # split 2 ways, 96 chains: 1,024
+    (1, 4096, 97, 0, 0), (4, 4000, 32, 0, 0), (4, 8192, 32, 0, 0), (32, 32768, 32, 0, 0),   # more chains
+    (1, 13952, 32, 1, 0), (1, 13953, 32, 2, 0), (1, 16384, 32, 2, 0), (1, 27905, 32, 3, 0),  # windows
+    (1, 20000, 24, 2, 0), (1, 20000, 23, 0, 0),                             # ... on 192 CUs, 184
+    (1, 30000, 16, 0, 0), (1, 60000, 8, 0, 0),
+    (2, 15200, 32, 3, 0), (2, 9000, 32, 1, 0), (1, 16384, 48, 2, 0), (1, 16384, 47, 0, 0),
+    (2, 8192, 48, 1, 1), (2, 16384, 48, 0, 0), (1, 16384, 96, 0, 0),        # split 2 ways: one window
+    (3, 4608, 32, 1, 1), (3, 4609, 32, 0, 0), (12, 12288, 2, 1, 0), (20, 20480, 1, 1, 0), (12, 30720, 2, 0, 0),
+    (0, 0, 32, 0, 0), (0, 5000, 32, 0, 0), (1, 0, 32, 0, 0), (-1, 5000, 32, 0, 0), (1, 5000, 0, 0, 0),
+])
+def test_prefill_dropin_route(lib, N, T, hv, windows, yields):
+    """The drop-in's choice between one kernel (0) and windows of two, and the batches that
+    yield the scratch to another stream, at the lines between them.  Without a GPU the CU
+    count defaults to 256."""
+    y = ctypes.c_int32(-1)
+    assert (lib.gdn_prefill_dropin_windows(N, T, hv, ctypes.byref(y)), y.value) == (windows, yields)
 
 
 def test_prefill_with_workspace_validates(lib):

@@ -3,10 +3,13 @@ prefill hand-offs live in each workgroup's LDS; a workspace belongs to one call;
 library's two scratch arrays are each ordered between launches by an event), so decode
 and prefill batches running concurrently on separate streams give the results of the
 same calls run one after another, bit for bit."""
+import ctypes
+
 import pytest
 import torch
 
 from gdn_kernel_amd import _lib, binding, workloads
+from gdn_kernel_amd.workloads import Heads
 from tests.gpu_util import say
 
 pytestmark = pytest.mark.gpu
@@ -101,3 +104,64 @@ def test_concurrent_streams_match_sequential(gpu):
     for i, ((o, s), (ro, rs)) in enumerate(zip(results, ref)):
         assert torch.equal(o, ro), f"stream {i}: output differs from the sequential run"
         assert torch.equal(s, rs), f"stream {i}: state differs from the sequential run"
+
+
+def test_short_batches_do_not_wait_for_other_streams(gpu):
+    """While one stream's launches hold the drop-in's scratch (6,000-token sequences at 8
+    v-heads, a quarter of the CUs), a 700-token sequence on another stream runs one kernel
+    beside them instead of waiting for them: it ends first, with the bits of the two-kernel
+    path.  (Six streams, as streams that share a hardware queue wait for each other.)"""
+    lib = _lib.load()
+    long = workloads.prefill_inputs([6000], Heads(4, 4, 8), seed=58, device=gpu, gate="slow", state_scale=0.5)
+    short = workloads.prefill_inputs([700], Heads(4, 4, 8), seed=59, device=gpu, gate="slow", state_scale=0.5)
+    yields = ctypes.c_int32()
+    assert lib.gdn_prefill_dropin_windows(1, 6000, 8, ctypes.byref(yields)) == 1 and yields.value == 0
+    assert lib.gdn_prefill_dropin_windows(1, 700, 8, ctypes.byref(yields)) == 1 and yields.value == 1
+
+    def held(stream):
+        h = ctypes.c_int32()
+        _lib.check(lib.gdn_prefill_dropin_held(ctypes.byref(h), stream.cuda_stream))
+        return h.value
+
+    def call(p, o, s):
+        binding.prefill_kernel(p["q"], p["k"], p["v"], p["state"], p["A_log"], p["a"], p["dt_bias"], p["b"],
+                               p["cu_seqlens"], p["scale"], o, s)
+
+    holder, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(6)]
+    ref = _outputs(short, 1)
+    call(short, *ref)                                # two kernels: nothing holds the scratch
+    outs = [_outputs(short, 1) for _ in others]
+    torch.cuda.synchronize()
+    for s, out in zip([holder, *others], [_outputs(short, 1), *outs]):   # a stream's first launch sets it up
+        with torch.cuda.stream(s):
+            call(short, *out)
+        torch.cuda.synchronize()
+        for x in out:
+            x.fill_(float("nan"))
+    lo, ls = _outputs(long, 1)
+    call(long, lo, ls)
+    want = lo.clone(), ls.clone()
+    torch.cuda.synchronize()
+    assert not any(held(s) for s in [holder, *others])
+    say("short batches beside a stream of long ones")
+    with torch.cuda.stream(holder):
+        for _ in range(40):
+            call(long, lo, ls)
+        end = torch.cuda.Event()
+        end.record()
+    ends = []
+    for s, (o, st) in zip(others, outs):
+        assert held(s) and not held(holder)
+        with torch.cuda.stream(s):
+            call(short, o, st)
+            ends.append(torch.cuda.Event())
+            ends[-1].record()
+    first = False
+    while not end.query():
+        first = first or any(e.query() for e in ends)
+    torch.cuda.synchronize()
+    assert first, "every short batch waited for the long ones"
+    assert not any(held(s) for s in others)
+    for o, st in outs:
+        assert torch.equal(o, ref[0]) and torch.equal(st, ref[1])
+    assert torch.equal(lo, want[0]) and torch.equal(ls, want[1])
