@@ -103,12 +103,18 @@ class _NoNative:
 
 
 def native():
-    """Load (once) and return the native module, bound to the library's entry points."""
+    """Load (once) and return the native module, bound to the library's entry points; for
+    now _NoNative where there is no library or no GPU build of torch, which the Python code
+    reports once it has checked the arguments."""
     global _native
     if _native is not None:
         return _native
-    lib = load()
     import torch
+    try:
+        lib = load()
+        device, stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+    except (ImportError, OSError, AttributeError):
+        return _NoNative
     try:
         from . import _native as mod
     except ImportError:
@@ -116,7 +122,7 @@ def native():
         return _native
     mod.bind(*(ctypes.cast(fn, c_void_p).value for fn in
                (lib.gdn_decode, lib.gdn_decode_pooled, lib.gdn_prefill, lib.gdn_prefill_with_workspace)),
-             torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+             device, stream)
     _native = mod
     return mod
 

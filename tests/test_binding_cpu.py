@@ -6,7 +6,35 @@ import numpy as np
 import pytest
 import torch
 
-from gdn_kernel_amd import binding, workloads
+from gdn_kernel_amd import _lib, binding, workloads
+
+
+@pytest.mark.parametrize("missing", ["library", "unloadable library", "GPU build of torch"])
+def test_arguments_are_checked_before_the_library(monkeypatch, tmp_path, missing):
+    """Bad arguments are reported as such where the library or torch's GPU functions are
+    missing; with the library missing, a call that passes its checks raises ImportError."""
+    monkeypatch.setattr(_lib, "_native", None)
+    if missing == "GPU build of torch":
+        monkeypatch.delattr(torch._C, "_cuda_getDevice")
+    else:
+        monkeypatch.setattr(_lib, "_lib", None)
+        monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "absent.so")
+        if missing == "unloadable library":
+            (tmp_path / "absent.so").write_bytes(b"not a library")
+    w = workloads.decode_inputs(2, seed=0, pool_slots=3)
+    p = workloads.prefill_inputs([3, 5], seed=0)
+    decode = [w[n] for n in ("q", "k", "v", "state", "A_log", "a", "dt_bias", "b", "scale")] + [w["v"]]
+    prefill = [p[n] for n in ("q", "k", "v", "state", "A_log", "a", "dt_bias", "b", "cu_seqlens", "scale")]
+    prefill += [p["v"], p["state"]]
+    for call in (lambda: binding.decode_kernel(*decode, w["state"]),
+                 lambda: binding.decode_pooled_kernel(*decode, w["state_indices"]),
+                 lambda: binding.prefill_kernel(*prefill),
+                 lambda: binding.prefill_kernel_with_workspace(*prefill, None)):
+        with pytest.raises(ValueError, match="GPU"):
+            call()
+    if missing == "library":
+        with pytest.raises(ImportError, match="not built"):
+            _lib.load()
 
 
 def test_binding_rejects_cpu_tensors():
