@@ -8,6 +8,7 @@ is the short call path of the Python entry points.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 from ctypes import c_double, c_int, c_int32, c_int64, c_void_p
 from pathlib import Path
 
@@ -105,7 +106,8 @@ class _NoNative:
 def native():
     """Load (once) and return the native module, bound to the library's entry points; for
     now _NoNative where there is no library or no GPU build of torch, which the Python code
-    reports once it has checked the arguments."""
+    reports once it has checked the arguments.  Without a native module the Python code takes
+    every call; one that does not load, or was built for another torch or library, raises."""
     global _native
     if _native is not None:
         return _native
@@ -115,11 +117,19 @@ def native():
         device, stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
     except (ImportError, OSError, AttributeError):
         return _NoNative
-    try:
-        from . import _native as mod
-    except ImportError:
+    if importlib.util.find_spec(f"{__package__}._native") is None:
         _native = _NoNative
         return _native
+    rebuild = "; run `python -m gdn_kernel_amd.build`"
+    try:
+        from . import _native as mod
+    except ImportError as e:
+        raise ImportError(f"the native module does not load{rebuild}") from e
+    for what, stamp, here in (("torch", "torch_version", str(torch.__version__)),
+                              ("the library", "library_build_id", lib.gdn_build_id().decode())):
+        if getattr(mod, stamp, None) != here:
+            raise ImportError(f"the native module was built for another version of {what} "
+                              f"({getattr(mod, stamp, None)}, here {here}){rebuild}")
     mod.bind(*(ctypes.cast(fn, c_void_p).value for fn in
                (lib.gdn_decode, lib.gdn_decode_pooled, lib.gdn_prefill, lib.gdn_prefill_with_workspace)),
              device, stream)

@@ -86,13 +86,22 @@ def build(verbose: bool = False, out: Path | None = None) -> Path:
 NATIVE_SOURCE = "gdn_torch.cpp"
 
 
+def native_digest(root: Path | None = None) -> str:
+    """Build id of the native module: as source_digest, over its source and the library's
+    build id (whose inputs hold the C header it is compiled against)."""
+    root = Path(root) if root is not None else PKG_DIR.parent
+    source = (root / "gdn_kernel_amd/csrc" / NATIVE_SOURCE).read_bytes()
+    return hashlib.sha256(source + b"\0" + source_digest(root).encode()).hexdigest()[:16]
+
+
 def native_path() -> Path:
     return PKG_DIR / f"_native{sysconfig.get_config_var('EXT_SUFFIX')}"
 
 
 def build_native(verbose: bool = False) -> Path:
     """Compile the native module of the Python entry points (host-only C++ over torch's
-    tensor headers; it takes the library's addresses at run time)."""
+    tensor headers; it takes the library's addresses at run time).  It is stamped with this
+    torch and these sources: _lib.native() refuses it beside another torch or library."""
     import torch
     root = Path(torch.__file__).resolve().parent
     out = native_path()
@@ -100,6 +109,8 @@ def build_native(verbose: bool = False) -> Path:
     cxx = os.environ.get("CXX") or shutil.which("g++") or "c++"
     cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           f'-DGDN_NATIVE_TORCH="{torch.__version__}"', f'-DGDN_NATIVE_LIBRARY="{source_digest()}"',
+           f'-DGDN_NATIVE_BUILD_ID="{native_digest()}"',
            "-isystem", str(root / "include"), "-isystem", str(root / "include/torch/csrc/api/include"),
            "-isystem", sysconfig.get_paths()["include"], str(CSRC / NATIVE_SOURCE),
            "-L", str(root / "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-o", str(tmp)]

@@ -13,24 +13,15 @@
 #include <cstdint>
 #include <initializer_list>
 
+#include "../../include/gdn_kernel_amd.h"
+
 namespace {
 
-using Decode = int (*)(const void*, const void*, const void*, const void*, const void*, const void*, const void*,
-                       const void*, double, void*, void*, int64_t, int32_t, int32_t, int32_t, int32_t, int32_t, void*);
-using Pooled = int (*)(const void*, const void*, const void*, void*, int64_t, const void*, const void*, const void*,
-                       const void*, const void*, double, void*, int64_t, int32_t, int32_t, int32_t, int32_t, int32_t,
-                       void*);
-using Prefill = int (*)(const void*, const void*, const void*, const void*, const void*, const void*, const void*,
-                        const void*, const void*, int32_t, int64_t, int64_t, double, void*, void*, int32_t, int32_t,
-                        int32_t, int32_t, int32_t, void*);
-using PrefillWs = int (*)(const void*, const void*, const void*, const void*, const void*, const void*, const void*,
-                          const void*, const void*, int32_t, int64_t, int64_t, double, void*, void*, int32_t, int32_t,
-                          int32_t, int32_t, int32_t, void*, int64_t, void*);
-
-Decode g_decode = nullptr;
-Pooled g_pooled = nullptr;
-Prefill g_prefill = nullptr;
-PrefillWs g_prefill_ws = nullptr;
+// The library's entry points (bind()).
+decltype(&gdn_decode) g_decode = nullptr;
+decltype(&gdn_decode_pooled) g_pooled = nullptr;
+decltype(&gdn_prefill) g_prefill = nullptr;
+decltype(&gdn_prefill_with_workspace) g_prefill_ws = nullptr;
 PyObject* g_device = nullptr;  // torch._C._cuda_getDevice
 PyObject* g_stream = nullptr;  // torch._C._cuda_getCurrentRawStream
 
@@ -48,7 +39,15 @@ bool is(const at::Tensor* t, at::ScalarType dtype, int device, std::initializer_
   return t->sizes().equals(at::IntArrayRef(shape)) && t->is_contiguous();
 }
 
-void* ptr(const at::Tensor* t) { return t == nullptr || t->numel() == 0 ? nullptr : t->data_ptr(); }
+// A tensor's memory, as whatever pointer an entry point takes.
+struct Ptr {
+  void* p;
+  template <class T>
+  operator T*() const {
+    return static_cast<T*>(p);
+  }
+};
+Ptr ptr(const at::Tensor* t) { return Ptr{t == nullptr || t->numel() == 0 ? nullptr : t->data_ptr()}; }
 
 // The scale argument: None (0, the default scale) or a number that is plainly a double.
 bool scale_of(PyObject* o, double* scale) {
@@ -101,9 +100,8 @@ PyObject* decode_impl(PyObject* const* o) {
       !is(out, kBf16, dev, {B, 1, Hv, dv}) || !is(ns, kF32, dev, {B, Hv, dv, dk}) || !scale_of(o[8], &scale) ||
       Hq > INT32_MAX || Hk > INT32_MAX || Hv > INT32_MAX || dk > INT32_MAX || dv > INT32_MAX || !stream_of(dev, &stream))
     return nullptr;
-  const void *pq = ptr(q), *pk = ptr(k), *pv = ptr(v), *ps = ptr(state), *pA = ptr(A_log), *pa = ptr(a), *pd = ptr(dt),
-             *pb = ptr(b);
-  void *po = ptr(out), *pn = ptr(ns);
+  const Ptr pq = ptr(q), pk = ptr(k), pv = ptr(v), ps = ptr(state), pA = ptr(A_log), pa = ptr(a), pd = ptr(dt),
+            pb = ptr(b), po = ptr(out), pn = ptr(ns);
   int rc;
   Py_BEGIN_ALLOW_THREADS
   rc = g_decode(pq, pk, pv, ps, pA, pa, pd, pb, scale, po, pn, B, int32_t(Hq), int32_t(Hk), int32_t(Hv), int32_t(dk),
@@ -130,9 +128,8 @@ PyObject* pooled_impl(PyObject* const* o) {
       !is(out, kBf16, dev, {B, 1, Hv, dv}) || !scale_of(o[8], &scale) || Hq > INT32_MAX || Hk > INT32_MAX ||
       Hv > INT32_MAX || dk > INT32_MAX || dv > INT32_MAX || !stream_of(dev, &stream))
     return nullptr;
-  const void *pq = ptr(q), *pk = ptr(k), *pv = ptr(v), *pi = ptr(idx), *pA = ptr(A_log), *pa = ptr(a), *pd = ptr(dt),
-             *pb = ptr(b);
-  void *pp = ptr(pool), *po = ptr(out);
+  const Ptr pq = ptr(q), pk = ptr(k), pv = ptr(v), pi = ptr(idx), pA = ptr(A_log), pa = ptr(a), pd = ptr(dt),
+            pb = ptr(b), pp = ptr(pool), po = ptr(out);
   int rc;
   Py_BEGIN_ALLOW_THREADS
   rc = g_pooled(pq, pk, pv, pp, slots, pi, pA, pa, pd, pb, scale, po, B, int32_t(Hq), int32_t(Hk), int32_t(Hv),
@@ -168,9 +165,8 @@ PyObject* prefill_impl(PyObject* const* o, bool with_workspace) {
       !is(out, kBf16, dev, {T, Hv, dv}) || !is(ns, kF32, dev, {N, Hv, dv, dk}) || !scale_of(o[9], &scale) ||
       Hq > INT32_MAX || Hk > INT32_MAX || Hv > INT32_MAX || dk > INT32_MAX || dv > INT32_MAX || !stream_of(dev, &stream))
     return nullptr;
-  const void *pq = ptr(q), *pk = ptr(k), *pv = ptr(v), *ps = ptr(state), *pA = ptr(A_log), *pa = ptr(a), *pd = ptr(dt),
-             *pb = ptr(b), *pc = cu->data_ptr();
-  void *po = ptr(out), *pn = ptr(ns), *pw = ptr(ws);
+  const Ptr pq = ptr(q), pk = ptr(k), pv = ptr(v), ps = ptr(state), pA = ptr(A_log), pa = ptr(a), pd = ptr(dt),
+            pb = ptr(b), pc = Ptr{cu->data_ptr()}, po = ptr(out), pn = ptr(ns), pw = ptr(ws);
   const int64_t wn = ws ? ws->size(0) : 0;
   int rc;
   Py_BEGIN_ALLOW_THREADS
@@ -223,10 +219,10 @@ PyObject* py_bind(PyObject*, PyObject* args) {
   unsigned long long d, dp, pf, pw;
   PyObject *device, *stream;
   if (!PyArg_ParseTuple(args, "KKKKOO", &d, &dp, &pf, &pw, &device, &stream)) return nullptr;
-  g_decode = reinterpret_cast<Decode>(static_cast<uintptr_t>(d));
-  g_pooled = reinterpret_cast<Pooled>(static_cast<uintptr_t>(dp));
-  g_prefill = reinterpret_cast<Prefill>(static_cast<uintptr_t>(pf));
-  g_prefill_ws = reinterpret_cast<PrefillWs>(static_cast<uintptr_t>(pw));
+  g_decode = reinterpret_cast<decltype(g_decode)>(static_cast<uintptr_t>(d));
+  g_pooled = reinterpret_cast<decltype(g_pooled)>(static_cast<uintptr_t>(dp));
+  g_prefill = reinterpret_cast<decltype(g_prefill)>(static_cast<uintptr_t>(pf));
+  g_prefill_ws = reinterpret_cast<decltype(g_prefill_ws)>(static_cast<uintptr_t>(pw));
   Py_INCREF(device);
   Py_INCREF(stream);
   Py_XSETREF(g_device, device);
@@ -248,4 +244,21 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Call path of the gdn_ke
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }
+// The module is compiled against one torch (it reads tensors in place) and one library (it
+// calls the addresses it is given); the loader compares all three stamps.
+#ifndef GDN_NATIVE_TORCH
+#define GDN_NATIVE_TORCH "unknown"
+#define GDN_NATIVE_LIBRARY "unknown"
+#define GDN_NATIVE_BUILD_ID "unknown"
+#endif
+PyMODINIT_FUNC PyInit__native(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m == nullptr) return nullptr;
+  if (PyModule_AddStringConstant(m, "torch_version", GDN_NATIVE_TORCH) != 0 ||
+      PyModule_AddStringConstant(m, "library_build_id", GDN_NATIVE_LIBRARY) != 0 ||
+      PyModule_AddStringConstant(m, "build_id", GDN_NATIVE_BUILD_ID) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

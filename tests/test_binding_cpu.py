@@ -1,6 +1,7 @@
 """CPU tests of the Python binding's argument checks and of the workload
 generators (no GPU; nothing is launched)."""
 import math
+import sys
 
 import numpy as np
 import pytest
@@ -35,6 +36,62 @@ def test_arguments_are_checked_before_the_library(monkeypatch, tmp_path, missing
     if missing == "library":
         with pytest.raises(ImportError, match="not built"):
             _lib.load()
+
+
+class _Module:
+    """A stand-in for the built native module."""
+
+    def __init__(self, **stamps):
+        self.bound = False
+        self.__dict__.update(stamps)
+
+    def bind(self, *args):
+        self.bound = True
+
+
+def _native_with(monkeypatch, module):
+    """_lib.native() where `module` (None: no file; an exception: its import raises it) is
+    the package's native module."""
+    monkeypatch.setattr(_lib, "_native", None)
+    spec = None if module is None else object()
+    monkeypatch.setattr(_lib.importlib.util, "find_spec", lambda name: spec)
+    package = sys.modules["gdn_kernel_amd"]
+    monkeypatch.delattr(package, "_native", raising=False)
+    monkeypatch.delitem(sys.modules, "gdn_kernel_amd._native", raising=False)
+    if isinstance(module, Exception):
+        class Finder:
+            @staticmethod
+            def find_spec(name, path=None, target=None):
+                if name == "gdn_kernel_amd._native":
+                    raise module
+        monkeypatch.setattr(sys, "meta_path", [Finder, *sys.meta_path])
+    elif module is not None:
+        monkeypatch.setattr(package, "_native", module, raising=False)
+    return _lib.native()
+
+
+def test_native_module_that_does_not_match_is_refused(monkeypatch):
+    """Only a missing native module leaves the calls to the Python code: one that does not
+    load, or that was built for another torch or another library (or before it was
+    stamped), raises."""
+    torch_version, library = str(torch.__version__), _lib.load().gdn_build_id().decode()
+    good = _Module(torch_version=torch_version, library_build_id=library)
+    assert _native_with(monkeypatch, good) is good and good.bound
+    assert _native_with(monkeypatch, None) is _lib._NoNative
+    with pytest.raises(ImportError, match="does not load"):
+        _native_with(monkeypatch, ImportError("undefined symbol"))
+    for stamps, what in (({}, "torch"), (dict(torch_version="1.0", library_build_id=library), "torch"),
+                         (dict(torch_version=torch_version, library_build_id="0" * 16), "library"),
+                         (dict(torch_version=torch_version), "library")):
+        with pytest.raises(ImportError, match=f"another version of .*{what}"):
+            _native_with(monkeypatch, _Module(**stamps))
+
+
+def test_native_module_is_built_from_these_sources():
+    from gdn_kernel_amd import _native, build
+    assert _native.build_id == build.native_digest()
+    assert _native.library_build_id == build.source_digest() == _lib.load().gdn_build_id().decode()
+    assert _native.torch_version == str(torch.__version__)
 
 
 def test_binding_rejects_cpu_tensors():
