@@ -177,9 +177,19 @@ def build_tvm_ffi(verbose: bool = False, paths: dict | None = None) -> dict:
     return built
 
 
-if __name__ == "__main__":
-    path = build(verbose="-v" in sys.argv)
-    print(f"built {path}")
-    print(f"built {build_native(verbose='-v' in sys.argv)}")
+def main(verbose: bool = False) -> None:
+    """Build the library, the native module and, where tvm-ffi is installed, its shims.  The
+    native module needs a host C++ compiler, Python's headers and torch; without them the
+    Python code takes its calls."""
+    print(f"built {build(verbose=verbose)}")
+    try:
+        print(f"built {build_native(verbose=verbose)}")
+    except (ImportError, OSError, RuntimeError) as e:
+        native_path().unlink(missing_ok=True)  # an earlier build's would not match the library
+        print(f"native module not built, calls take the Python path: {e}")
     for op, p in build_tvm_ffi(verbose=True).items():
         print(f"built {p} (TVM-FFI `kernel`, {op})")
+
+
+if __name__ == "__main__":
+    main(verbose="-v" in sys.argv)

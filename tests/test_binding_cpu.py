@@ -94,6 +94,28 @@ def test_native_module_is_built_from_these_sources():
     assert _native.torch_version == str(torch.__version__)
 
 
+@pytest.mark.parametrize("cxx", ["absent", "failing"])
+def test_build_without_a_host_compiler(monkeypatch, tmp_path, capsys, cxx):
+    """Without a working host compiler `python -m gdn_kernel_amd.build` still builds the
+    library and goes on to the TVM-FFI shims; a native module of an earlier build, which
+    would not match, goes."""
+    from gdn_kernel_amd import build
+    compiler = tmp_path / "c++"
+    if cxx == "failing":
+        compiler.write_text("#!/bin/sh\nexit 1\n")
+        compiler.chmod(0o755)
+    monkeypatch.setenv("CXX", str(compiler))
+    (tmp_path / "_native.so").write_bytes(b"")
+    shims = []
+    monkeypatch.setattr(build, "build", lambda verbose: tmp_path / "lib.so")
+    monkeypatch.setattr(build, "native_path", lambda: tmp_path / "_native.so")
+    monkeypatch.setattr(build, "build_tvm_ffi", lambda verbose: shims.append(1) or {})
+    build.main()
+    out = capsys.readouterr().out
+    assert "lib.so" in out and "native module not built" in out and shims == [1]
+    assert not (tmp_path / "_native.so").exists()
+
+
 def test_binding_rejects_cpu_tensors():
     w = workloads.decode_inputs(2, seed=0)
     out = torch.empty_like(w["v"])
