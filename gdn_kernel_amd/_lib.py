@@ -59,6 +59,9 @@ SIGNATURES = {
                                         c_int64] + _HEADS + [c_int32, _P], c_int),
     "gdn_prefill_fault_injection": ([_P] * 8 + [_P, c_int32, c_int64, c_int64, c_double, _P, _P]
                                     + _HEADS + [c_int32, c_int32, _P, _P], c_int),
+    "gdn_prefill_fault_injection_with_workspace": (
+        [_P] * 8 + [_P, c_int32, c_int64, c_int64, c_double, _P, _P] + _HEADS
+        + [_P, c_int64, c_int32, c_int32, _P, _P], c_int),
     "gdn_prefill_dropin_windows": ([c_int64, c_int64, c_int32, ctypes.POINTER(c_int32)], c_int64),
     "gdn_prefill_dropin_held": ([ctypes.POINTER(c_int32), _P], c_int),
 }

@@ -289,6 +289,13 @@ int prefill_impl(const gdn_bf16* q, const gdn_bf16* k, const gdn_bf16* v, const 
   return device_status(e, "gdn_prefill launch");
 }
 
+int check_hooks(int32_t spin_limit, int32_t ready_chunks) {
+  if (spin_limit < 0 || ready_chunks < 0)
+    return fail(GDN_ERR_INVALID_ARGUMENT, "spin_limit and ready_chunks must be >= 0 (got %d, %d)", spin_limit,
+                ready_chunks);
+  return ok();
+}
+
 int check_variant(int32_t variant) {
   if (variant < 0 || variant >= gdn::kDecodeVariants)
     return fail(GDN_ERR_INVALID_ARGUMENT, "variant must be in [0, %d) (got %d)", gdn::kDecodeVariants, variant);
@@ -376,6 +383,18 @@ int gdn_decode_pool_conflicts(uint64_t* count, int32_t reset) {
   return device_status(gdn::decode_pool_conflicts(count, reset != 0), "gdn_decode_pool_conflicts");
 }
 
+int gdn_prefill_fault_injection_with_workspace(
+    const gdn_bf16* q, const gdn_bf16* k, const gdn_bf16* v, const float* state, const float* A_log,
+    const gdn_bf16* a, const float* dt_bias, const gdn_bf16* b, const void* cu_seqlens, int32_t cu_seqlens_dtype,
+    int64_t num_seqs, int64_t total_tokens, double scale, gdn_bf16* output, float* new_state, int32_t num_q_heads,
+    int32_t num_k_heads, int32_t num_v_heads, int32_t head_dim_k, int32_t head_dim_v, void* workspace,
+    int64_t workspace_bytes, int32_t spin_limit, int32_t ready_chunks, uint32_t* aborts, void* stream) {
+  GDN_TRY(check_hooks(spin_limit, ready_chunks));
+  return prefill_impl(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, cu_seqlens_dtype, num_seqs, total_tokens,
+                      scale, output, new_state, num_q_heads, num_k_heads, num_v_heads, head_dim_k, head_dim_v,
+                      spin_limit, ready_chunks, aborts, workspace, workspace_bytes, stream);
+}
+
 int64_t gdn_prefill_dropin_windows(int64_t num_seqs, int64_t total_tokens, int32_t num_v_heads, int32_t* yields) {
   gdn::PrefillRoute r = {0, false};
   if (num_seqs > 0 && num_seqs <= INT32_MAX && num_v_heads > 0)
@@ -422,9 +441,7 @@ int gdn_prefill_fault_injection(const gdn_bf16* q, const gdn_bf16* k, const gdn_
                                 int32_t num_q_heads, int32_t num_k_heads, int32_t num_v_heads, int32_t head_dim_k,
                                 int32_t head_dim_v, int32_t spin_limit, int32_t ready_chunks, uint32_t* aborts,
                                 void* stream) {
-  if (spin_limit < 0 || ready_chunks < 0)
-    return fail(GDN_ERR_INVALID_ARGUMENT, "spin_limit and ready_chunks must be >= 0 (got %d, %d)", spin_limit,
-                ready_chunks);
+  GDN_TRY(check_hooks(spin_limit, ready_chunks));
   return prefill_impl(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, cu_seqlens_dtype, num_seqs, total_tokens,
                       scale, output, new_state, num_q_heads, num_k_heads, num_v_heads, head_dim_k, head_dim_v,
                       spin_limit, ready_chunks, aborts, nullptr, 0, stream);

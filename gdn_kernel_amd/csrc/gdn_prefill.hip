@@ -1527,7 +1527,7 @@ __device__ __forceinline__ void loader_loop(PrefillSmem& sm, const PrefillArgs& 
       if (seg < V::VSEG)
         *reinterpret_cast<u32x4*>(sm.V + (seg / (V::ROWS / 8)) * VSTR + 8 * (seg % (V::ROWS / 8))) = fv[it];
     }
-    signal_count(sm, kReady, lane);
+    if (!V::kHooks || p.ready_chunks <= 0 || t < p.ready_chunks) signal_count(sm, kReady, lane);
     // The next chunks' loads go out after the hand-off.  Issued before it, the
     // waits for this tick's registers (loaded a tick earlier) would also wait for
     // them: the K/Q loads are conditional, so the compiler cannot count them and
@@ -2242,7 +2242,12 @@ struct __align__(16) StateSmem {
   int sync[16];                          // hand-off counters
   int seq;
 };
-static_assert(sizeof(StateSmem) <= 160 * 1024);
+// With testing hooks: as in PrefillSmem.
+struct HookedStateSmem : StateSmem {
+  int spin_limit;
+  unsigned* aborts;
+};
+static_assert(sizeof(HookedStateSmem) <= 160 * 1024);
 
 // Hand-offs of the state pass.  kAbort as in the other kernels.  "Loaded" and "output read"
 // count by chunk parity: a helper wave may be a chunk ahead of another, and with one counter
@@ -2274,7 +2279,8 @@ constexpr int kStateLoaders = 256;  // helper threads (four waves)
 //   fragments, which no other wave reads: they go straight into registers.
 // A wave that issues loads while the memory queue is full stalls (about 800 cycles a chunk);
 // here that delays no consumer.
-__device__ __forceinline__ void state_helper(StateSmem& sm, const PrefillArgs& p, const u32x4* tiles, int64_t s0,
+template <bool kHooks, class Smem>
+__device__ __forceinline__ void state_helper(Smem& sm, const PrefillArgs& p, const u32x4* tiles, int64_t s0,
                                              int64_t s1, int nchunks, int h, int hq, int hk, int row0, int w,
                                              int lane0) {
   const int pt = 64 * w + lane0;
@@ -2313,7 +2319,7 @@ __device__ __forceinline__ void state_helper(StateSmem& sm, const PrefillArgs& p
     for (int it = 0; it < 3; ++it) *reinterpret_cast<u32x4*>(sm.T[b] + 8 * (pt + kStateLoaders * it)) = r.t[it];
     if (pt < kGateUnits) *reinterpret_cast<u32x4*>(sm.gate[b] + 4 * pt) = r.g;
     if (pt < 2 * C) *reinterpret_cast<u32x4*>(sm.V[b] + 8 * pt) = r.v;
-    signal_count(sm, kLoaded + b, lane);
+    if (!kHooks || p.ready_chunks <= 0 || t < p.ready_chunks) signal_count(sm, kLoaded + b, lane);
   };
   // The output block's own operands: Q rows, P fragments and e^gamma of its tokens.
   RowFrags qf;
@@ -2330,7 +2336,7 @@ __device__ __forceinline__ void state_helper(StateSmem& sm, const PrefillArgs& p
   };
   // o^T = scale e^gamma (S Q^T) + v_new^T (scale P)^T of chunk t, tokens 16 ct .. +15.
   auto output = [&](int t, int sbuf, int lane) {
-    wait_count<false>(sm, kVnewIn, 4 * (t + 1));
+    wait_count<kHooks>(sm, kVnewIn, 4 * (t + 1));
     uint4 Sh[4];
     uint2 vn[4];
 #pragma unroll
@@ -2368,7 +2374,7 @@ __device__ __forceinline__ void state_helper(StateSmem& sm, const PrefillArgs& p
     asm volatile("" : "+v"(lane));
     // Chunk t + 2 first: the consumers take it sooner than they miss this output.
     if (t + 2 <= last) {
-      wait_count<false>(sm, kChunkRead, 4 * (t + 1));
+      wait_count<kHooks>(sm, kChunkRead, 4 * (t + 1));
       stage(t + 2, r, lane);
     }
     output(t, sbuf, lane);
@@ -2405,7 +2411,8 @@ __device__ __forceinline__ void state_helper(StateSmem& sm, const PrefillArgs& p
 // prep kernel included: 108 us a call; with K, Q, T~ and P all staged through the LDS and the
 // outputs formed by the consumers 121.5; with the consumers loading their own K, Q and P
 // rows into registers 152 (their loads stall behind the loaders').
-__device__ __forceinline__ void state_consumer(StateSmem& sm, const PrefillArgs& p, int64_t s0, int64_t s1, int nchunks,
+template <bool kHooks, class Smem>
+__device__ __forceinline__ void state_consumer(Smem& sm, const PrefillArgs& p, int64_t s0, int64_t s1, int nchunks,
                                                int wave, int lane0, f32x4 (&S)[2]) {
   const int ct = wave;  // this wave's 16-token block and 32-column block
   // K^T operand base of column blocks 2 ct, 2 ct + 1 (kt_bases with kt / 2 = ct).
@@ -2434,7 +2441,7 @@ __device__ __forceinline__ void state_consumer(StateSmem& sm, const PrefillArgs&
     signal_count(sm, kStateIn, lane);
   };
   put_state(0, lane0);
-  wait_count<false>(sm, kLoaded, 4);
+  wait_count<kHooks>(sm, kLoaded, 4);
   read_ahead(0, lane0);
   int sbuf = 0;  // t % 3
   for (int t = 0; t < nchunks; ++t) {
@@ -2447,7 +2454,7 @@ __device__ __forceinline__ void state_consumer(StateSmem& sm, const PrefillArgs&
     // The chunk-start state; the next chunk's buffers looked at in the same read (the last
     // chunk looks at its own).
     const int tn = min(t + 1, nchunks - 1);
-    const bool loaded = wait_count_peek<false>(sm, kStateIn, 4 * (t + 1), kLoaded + (tn & 1), 4 * ((tn >> 1) + 1));
+    const bool loaded = wait_count_peek<kHooks>(sm, kStateIn, 4 * (t + 1), kLoaded + (tn & 1), 4 * ((tn >> 1) + 1));
     uint4 Sh[4], Sl[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
@@ -2483,7 +2490,7 @@ __device__ __forceinline__ void state_consumer(StateSmem& sm, const PrefillArgs&
     signal_count(sm, kYIn, lane);
     // All of Y; the helpers done with the v_new (of chunk t - 2) and the state (before it)
     // whose buffers this chunk rewrites, looked at in the same read.
-    const bool out_read = wait_count_peek<false>(sm, kYIn, 4 * (t + 1), kOutRead + b, 4 * (t >> 1));
+    const bool out_read = wait_count_peek<kHooks>(sm, kYIn, 4 * (t + 1), kOutRead + b, 4 * (t >> 1));
     uint4 Y[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) Y[c] = sm.Y[c][lane];
@@ -2525,7 +2532,7 @@ __device__ __forceinline__ void state_consumer(StateSmem& sm, const PrefillArgs&
         Vn[c] = mfma(tl, Yh[js], Vn[c]);
       }
     }
-    if (!out_read) wait_count<false>(sm, kOutRead + b, 4 * (t >> 1));
+    if (!out_read) wait_count<kHooks>(sm, kOutRead + b, 4 * (t >> 1));
 
     // 3: columns 32ct .. 32ct + 31 of S = e^{gamma_last} S + sum_c K[c]^T (d_c v_new[c]).
     uint4 Uh[2], Ul[2];
@@ -2546,7 +2553,7 @@ __device__ __forceinline__ void state_consumer(StateSmem& sm, const PrefillArgs&
     sm.Vn[b][ct][lane] = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     signal_count(sm, kVnewIn, lane);
     if (t + 1 < nchunks) {
-      if (!loaded) wait_count<false>(sm, kLoaded + (tn & 1), 4 * ((tn >> 1) + 1));
+      if (!loaded) wait_count<kHooks>(sm, kLoaded + (tn & 1), 4 * ((tn >> 1) + 1));
       read_ahead(tn, lane);
     }
   }
@@ -2556,9 +2563,10 @@ __device__ __forceinline__ void state_consumer(StateSmem& sm, const PrefillArgs&
 // placed as in gdn_prefill_kernel with F = 8: the slices of a GQA pair of chains share an
 // XCD.  Waves 0-3 are consumers, 4-7 loaders.
 constexpr int kStateSlices = 8;
+template <bool HOOKS>
 __global__ __launch_bounds__(512) void gdn_prefill_state_kernel(PrefillArgs p) {
   constexpr int F = kStateSlices;
-  __shared__ StateSmem sm;
+  __shared__ std::conditional_t<HOOKS, HookedStateSmem, StateSmem> sm;
   const int tid = threadIdx.x;
   const int lane0 = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2574,13 +2582,19 @@ __global__ __launch_bounds__(512) void gdn_prefill_state_kernel(PrefillArgs p) {
   const int64_t s0 = sr.s0, s1 = sr.s1;
   const int nchunks = int((s1 - s0 + C - 1) / C);
   if (tid < 16) sm.sync[tid] = 0;
+  if constexpr (HOOKS) {
+    if (tid == 0) {
+      sm.spin_limit = p.spin_limit > 0 ? p.spin_limit : kSpinLimit;
+      sm.aborts = p.aborts;
+    }
+  }
   __syncthreads();  // counters cleared; pick_sequence's scratch read
   const u32x4* tiles =
       reinterpret_cast<const u32x4*>(p.tiles) + (int64_t(chunks_before(p, seq, lane0)) * p.Hv + h) * kTileImage;
 
   if (wave >= 4) {
     if (nchunks > 0) {
-      state_helper(sm, p, tiles, s0, s1, nchunks, h, hq, hk, row0, wave - 4, lane0);
+      state_helper<HOOKS>(sm, p, tiles, s0, s1, nchunks, h, hq, hk, row0, wave - 4, lane0);
       if (aborted(sm)) {
         // A hand-off wait gave up: NaN over the slice's outputs (wave w: tokens
         // s0 + 16 (4m + w) + lane % 16).
@@ -2604,7 +2618,7 @@ __global__ __launch_bounds__(512) void gdn_prefill_state_kernel(PrefillArgs p) {
     if (p.state) S[j] = ld4(p.state + srow + 16 * j);
   }
   if (nchunks > 0) {
-    state_consumer(sm, p, s0, s1, nchunks, wave, lane0, S);
+    state_consumer<HOOKS>(sm, p, s0, s1, nchunks, wave, lane0, S);
     if (aborted(sm)) {  // a hand-off wait gave up: NaN over the slice's state
       const float nan = __builtin_nanf("");
       S[0] = S[1] = f32x4{nan, nan, nan, nan};
@@ -3080,8 +3094,7 @@ PrefillRoute dropin_route(int N, int64_t T, int Hv) {
 // anyway.
 hipError_t launch_prefill_dropin(const PrefillArgs& a, hipStream_t stream) {
   const PrefillRoute r = dropin_route(a.N, a.T, a.Hv);
-  if (r.windows == 0 || a.spin_limit != 0 || a.ready_chunks != 0 || a.aborts != nullptr || a.tiles != nullptr)
-    return launch_prefill(a, stream);
+  if (r.windows == 0) return launch_prefill(a, stream);
   hipError_t e = hipSuccess;
   if (stream_capturing(stream, &e)) return launch_prefill(a, stream);
   if (e != hipSuccess) return e;
@@ -3181,6 +3194,22 @@ int64_t prefill_workspace_bytes(int N, int64_t T, int Hv) {
 }
 
 namespace {
+// Launches that use the testing hooks get kernels with the hooks compiled in;
+// production launches keep them out of the device code.
+bool has_hooks(const PrefillArgs& a) { return a.spin_limit != 0 || a.ready_chunks != 0 || a.aborts != nullptr; }
+
+template <bool HOOKS>
+hipError_t launch_state(const PrefillArgs& a, hipStream_t stream, hipEvent_t done) {
+  const int64_t chains = int64_t(a.N) * a.Hv;
+  const dim3 grid(unsigned((chains + 15) / 16 * 16 * kStateSlices)), block(512);
+  if (done != nullptr) {
+    hipExtLaunchKernelGGL(gdn_prefill_state_kernel<HOOKS>, grid, block, 0, stream, nullptr, done, 0, a);
+  } else {
+    hipLaunchKernelGGL(gdn_prefill_state_kernel<HOOKS>, grid, block, 0, stream, a);
+  }
+  return hipGetLastError();
+}
+
 // The two-kernel path with room for `slots` chunk images a v-head (at least N), in
 // plan_windows' windows, each a prep kernel and a state pass that takes the state up where
 // the window before left it, in new_state: the same operations in the same order.  A window
@@ -3194,6 +3223,7 @@ hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t 
   PrefillArgs b = a;
   b.prep_slots = int(tc + a.N - 1 < a.N * w ? tc + a.N - 1 : a.N * w);
   const int64_t chains = int64_t(a.N) * a.Hv;
+  const bool hooks = has_hooks(a);
   for (int64_t i = 0; i < windows; ++i) {
     if (windows > 1) {
       b.win_begin = i * w * C;
@@ -3204,18 +3234,14 @@ hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const hipEvent_t last = i + 1 == windows ? done : nullptr;
+    // (The testing hooks reach this path through a workspace, which no batch split 2 ways uses.)
     if (split_factor(chains) == 2) {
       e = launch_variant<Variant<4, 1, false, true>>(b, stream, last);
     } else if (split_factor(chains) == 4) {
-      e = launch_variant<Variant<2, 1, false, true>>(b, stream, last);
+      e = hooks ? launch_variant<Variant<2, 1, true, true>>(b, stream, last)
+                : launch_variant<Variant<2, 1, false, true>>(b, stream, last);
     } else {
-      const dim3 sgrid(unsigned((chains + 15) / 16 * 16 * kStateSlices)), sblock(512);
-      if (last != nullptr) {
-        hipExtLaunchKernelGGL(gdn_prefill_state_kernel, sgrid, sblock, 0, stream, nullptr, last, 0, b);
-      } else {
-        hipLaunchKernelGGL(gdn_prefill_state_kernel, sgrid, sblock, 0, stream, b);
-      }
-      e = hipGetLastError();
+      e = hooks ? launch_state<true>(b, stream, last) : launch_state<false>(b, stream, last);
     }
     if (e != hipSuccess) return e;
     b.state = a.new_state;
@@ -3226,9 +3252,9 @@ hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t 
 
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream, hipEvent_t done) {
   const int F = split_factor(int64_t(a.N) * a.Hv);
-  // Launches that use the testing hooks get kernels with the hooks compiled in;
-  // production launches keep them out of the device code.
-  if (a.spin_limit != 0 || a.ready_chunks != 0 || a.aborts != nullptr) {
+  if (a.tiles != nullptr && prefill_workspace_bytes(a.N, a.T, a.Hv) > 0)
+    return launch_two_kernels(a, stream, a.N * ((a.T + C - 1) / C), done);
+  if (has_hooks(a)) {
     if (persistent_batch(a)) return launch_persistent<PersistVariant<true>>(a, stream);
     switch (F) {
       case 1: return launch_variant<SplitVariant1<true>>(a, stream);
@@ -3237,8 +3263,6 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream, hipEvent_t d
       default: return launch_variant<SplitVariant8<true>>(a, stream);
     }
   }
-  if (a.tiles != nullptr && prefill_workspace_bytes(a.N, a.T, a.Hv) > 0)
-    return launch_two_kernels(a, stream, a.N * ((a.T + C - 1) / C), done);
   // Split chains use 16-row consumer waves (VT = 1), whose per-chunk chain is
   // shorter than a 32-row wave's.  Unsplit chains (F = 1) keep four 32-row waves:
   // eight 16-row waves and the four producers would exceed the register file.

@@ -40,6 +40,18 @@ int gdn_prefill_fault_injection(const gdn_bf16* q, const gdn_bf16* k, const gdn_
                                 int32_t ready_chunks, uint32_t* aborts, void* stream);
 
 /*
+ * gdn_prefill_with_workspace with the same hooks (chunk ready: a chunk's images, K and V
+ * staged by the state pass's helper or loader waves).
+ */
+int gdn_prefill_fault_injection_with_workspace(
+    const gdn_bf16* q, const gdn_bf16* k, const gdn_bf16* v, const float* state, const float* A_log,
+    const gdn_bf16* a, const float* dt_bias, const gdn_bf16* b, const void* cu_seqlens,
+    int32_t cu_seqlens_dtype, int64_t num_seqs, int64_t total_tokens, double scale, gdn_bf16* output,
+    float* new_state, int32_t num_q_heads, int32_t num_k_heads, int32_t num_v_heads,
+    int32_t head_dim_k, int32_t head_dim_v, void* workspace, int64_t workspace_bytes,
+    int32_t spin_limit, int32_t ready_chunks, uint32_t* aborts, void* stream);
+
+/*
  * How gdn_prefill runs a batch outside graph capture: the number of windows of the
  * two-kernel path (0: one kernel).  *yields (if not null) is 1 for a batch that runs one
  * kernel all the same while a launch of another stream holds the library's scratch;

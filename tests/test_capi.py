@@ -176,6 +176,9 @@ def test_prefill_fault_injection_rejects(lib, kw, code, frag):
     for spin, ready in ((-1, 0), (0, -2)):
         assert lib.gdn_prefill_fault_injection(*pre_args(), spin, ready, None, None) == INVALID
         assert "spin_limit" in _lib.last_error()
+        assert lib.gdn_prefill_fault_injection_with_workspace(*pre_args(), FAKE, 1 << 40, spin, ready, None,
+                                                              None) == INVALID
+        assert "spin_limit" in _lib.last_error()
 
 
 def test_prefill_workspace_size(lib):

@@ -304,8 +304,10 @@ def test_prefill_no_tokens(gpu, with_state):
     assert torch.equal(ns.cpu(), ref)
 
 
-def _prefill_fault_injection(p, gpu, spin_limit, ready_chunks):
-    """gdn_prefill_fault_injection through the C ABI; returns (output, new_state, aborts)."""
+def _prefill_fault_injection(p, gpu, spin_limit, ready_chunks, workspace=False):
+    """gdn_prefill_fault_injection (one kernel), or with `workspace`
+    gdn_prefill_fault_injection_with_workspace, through the C ABI; returns (output,
+    new_state, aborts)."""
     d = {k: (v.to(gpu) if isinstance(v, torch.Tensor) else v) for k, v in p.items()}
     T, Hq = d["q"].shape[0], d["q"].shape[1]
     Hk, Hv = d["k"].shape[1], d["v"].shape[1]
@@ -316,12 +318,19 @@ def _prefill_fault_injection(p, gpu, spin_limit, ready_chunks):
     aborts = torch.zeros(1, device=gpu, dtype=torch.int32)
     cu_code = _lib.GDN_INDEX_INT32 if cu.dtype == torch.int32 else _lib.GDN_INDEX_INT64
     ptr = lambda t: None if t is None else t.data_ptr()
-    rc = _lib.load().gdn_prefill_fault_injection(
-        ptr(d["q"]), ptr(d["k"]), ptr(d["v"]), ptr(d["state"]), ptr(d["A_log"]), ptr(d["a"]),
-        ptr(d["dt_bias"]), ptr(d["b"]), cu.data_ptr(), cu_code, N, T, d["scale"], ptr(out), ptr(ns),
-        Hq, Hk, Hv, 128, 128, spin_limit, ready_chunks, ptr(aborts),
-        torch.cuda.current_stream(gpu).cuda_stream)
-    _lib.check(rc)
+    args = [ptr(d["q"]), ptr(d["k"]), ptr(d["v"]), ptr(d["state"]), ptr(d["A_log"]), ptr(d["a"]),
+            ptr(d["dt_bias"]), ptr(d["b"]), cu.data_ptr(), cu_code, N, T, d["scale"], ptr(out), ptr(ns),
+            Hq, Hk, Hv, 128, 128]
+    hooks = [spin_limit, ready_chunks, ptr(aborts), torch.cuda.current_stream(gpu).cuda_stream]
+    lib = _lib.load()
+    if workspace:
+        nbytes = lib.gdn_prefill_workspace_size(N, T, Hv)
+        assert nbytes > 0, "expected a batch that the two-kernel path serves"
+        ws = torch.full((nbytes,), 0xFF, device=gpu, dtype=torch.uint8)
+        _lib.check(lib.gdn_prefill_fault_injection_with_workspace(*args, ptr(ws), nbytes, *hooks))
+        torch.cuda.synchronize()
+    else:
+        _lib.check(lib.gdn_prefill_fault_injection(*args, *hooks))
     return out, ns, aborts
 
 
@@ -509,6 +518,39 @@ def test_prefill_bounded_waits(gpu, heads, split):
     say("prefill bounded waits: a normal launch afterwards")
     o3, s3 = run_prefill(p, gpu)
     torch.cuda.synchronize()
+    assert torch.equal(o3, o1) and torch.equal(s3, s1)
+    assert binding.prefill_giveups() == 0
+
+
+@pytest.mark.giveups_expected
+@pytest.mark.parametrize("heads,split", [(Heads(8, 8, 16), 4), (Heads(4, 4, 8), 8)])
+def test_prefill_two_kernels_bounded_waits(gpu, heads, split):
+    """The hand-off failure path of the state pass (48 chains split 4 ways: the general
+    kernel's loader variant; 24 split 8 ways: the state kernel), forced from the host as in
+    test_prefill_bounded_waits: with the waves that stage the chunks signalling only the
+    first, every workgroup of a sequence of two or more chunks gives up, is counted, and
+    leaves NaN in every output and final-state element it owns; the one-chunk sequence is
+    untouched, and with the hooks off, before and after, nothing gives up."""
+    lens = [300, 130, 40]             # 5, 3 and 1 chunks
+    p = workloads.prefill_inputs(lens, heads, seed=23, gate="slow", state_scale=0.5)
+    binding.prefill_giveups(reset=True)
+    say(f"prefill two kernels bounded waits, split {split}: hooks off")
+    o1, s1 = _prefill_capi(p, gpu, workspace=True)
+    o0, s0, a0 = _prefill_fault_injection(p, gpu, 0, 0, workspace=True)
+    assert int(a0.item()) == 0 and binding.prefill_giveups() == 0
+    assert torch.equal(o0, o1) and torch.equal(s0, s1)
+    say("prefill two kernels bounded waits: chunk-ready signals stop after chunk 0, 2000-poll limit")
+    o2, s2, a2 = _prefill_fault_injection(p, gpu, 2000, 1, workspace=True)
+    waiting_wgs = 2 * heads.hv * split  # sequences with >= 2 chunks x v-heads x workgroups per chain
+    n = int(a2.item())
+    assert waiting_wgs <= n <= waiting_wgs * 8, n
+    assert binding.prefill_giveups(reset=True) == n, "the device counter must see every give-up"
+    s, e = sum(lens[:2]), sum(lens)
+    assert torch.isnan(o2[:s].float()).all() and torch.isnan(s2[:2]).all(), \
+        "outputs and states of the sequences whose waits gave up must be NaN"
+    assert torch.equal(o2[s:e], o1[s:e]) and torch.equal(s2[2], s1[2])
+    say("prefill two kernels bounded waits: a normal launch afterwards")
+    o3, s3 = _prefill_capi(p, gpu, workspace=True)
     assert torch.equal(o3, o1) and torch.equal(s3, s1)
     assert binding.prefill_giveups() == 0
 
