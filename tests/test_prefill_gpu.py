@@ -1,5 +1,7 @@
 """GPU parity tests of the varlen chunked prefill kernel (through the C ABI)
 against the CPU oracle, plus size-independent properties at full size."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -179,16 +181,20 @@ def test_prefill_edge_gates(gpu, lens, state_scale):
     (its linear branch), saturated beta (b = +-12, +-30) and A_log from -12 (no decay) to
     4 (e^4 per unit of softplus: the state is wiped by any token with a > 20), per v-head.
     Fast-decay chunks take the log-gate sums to ~1e5 in magnitude while the decays that
-    matter come from differences below 1e2: the kernel sums them in fp64.  Five sequences
-    (160 chains) run as one kernel; the single 300-token sequence (32 chains) on the
-    two-kernel path."""
+    matter come from differences below 1e2: the kernel sums them in fp64.  Both batches run
+    as one kernel; the single 300-token sequence (32 chains) also on the two-kernel path,
+    with a workspace."""
     say(f"prefill edge gates lens={lens} state_scale={state_scale}")
     p = workloads.prefill_inputs(lens, seed=41, gate="edge", state_scale=state_scale)
     x = to_numpy(p["a"]) + to_numpy(p["dt_bias"])
     assert (x > 20).any() and (np.abs(to_numpy(p["b"])) >= 12).any()
+    assert _dropin_windows(p)[0] == 0
     o_ref, s_ref = oracle_prefill(p)
     out, ns = run_prefill(p, gpu)
     torch.cuda.synchronize()
+    if len(lens) == 1:
+        o2, s2 = _prefill_capi(p, gpu, workspace=True)
+        assert torch.equal(o2, out) and torch.equal(s2, ns), "workspace path differs from one kernel"
     assert_close(host(out), o_ref, OUT_RTOL, OUT_ATOL, "output")
     assert_close(host(ns), s_ref, STATE_RTOL, STATE_ATOL, "new_state")
 
@@ -209,6 +215,7 @@ def test_prefill_no_decay_precision_envelope(gpu, lens, heads):
     say(f"prefill no-decay precision envelope lens={lens} heads={heads}")
     p = workloads.prefill_inputs(lens, heads, seed=43, gate="edge", state_scale=0.5)
     p["A_log"] = torch.full((heads.hv,), -12.0)
+    assert _dropin_windows(p) == (1, 0)
     o_ref, s_ref = oracle_prefill(p)
     out, ns = run_prefill(p, gpu)
     torch.cuda.synchronize()
@@ -334,6 +341,15 @@ def _prefill_fault_injection(p, gpu, spin_limit, ready_chunks, workspace=False):
     return out, ns, aborts
 
 
+def _dropin_windows(p):
+    """How gdn_prefill runs the batch: (windows of the two-kernel path, 0 for one kernel;
+    whether it yields to another stream)."""
+    yields = ctypes.c_int32(-1)
+    n = _lib.load().gdn_prefill_dropin_windows(p["cu_seqlens"].numel() - 1, p["q"].shape[0], p["v"].shape[1],
+                                               ctypes.byref(yields))
+    return n, yields.value
+
+
 def _prefill_capi(p, gpu, workspace, ws=None, nbytes=None):
     """gdn_prefill, or gdn_prefill_with_workspace with a workspace of exactly the
     reported size (or the given buffer), through the C ABI; returns (output, new_state)."""
@@ -369,25 +385,26 @@ def _prefill_capi(p, gpu, workspace, ws=None, nbytes=None):
     ([150, 64, 7, 0], Heads(4, 4, 8)),           # ragged, an empty sequence
     ([150, 64, 7, 0, 65, 200], Heads(4, 4, 8)),  # 48 chains: split 4 ways (two 16-row consumers)
     ([130, 2100], Heads(16, 16, 32)),            # 64 chains, split 4 ways
-    ([1, 2, 63, 64, 129], Heads(2, 2, 4)),       # boundary lengths (chunk runs of 1 in the prep)
-    ([700, 1300], Heads(8, 8, 16)),              # runs of several chunks per prep workgroup
+    ([1, 2, 63, 64, 129], Heads(2, 2, 4)),       # boundary lengths
+    ([700, 1300], Heads(8, 8, 16)),              # 32 chains of many chunks
     ([1000], Heads(16, 8, 32)),                  # distinct q and k head ratios, split 8 ways
-    ([3000, 2000], Heads(16, 16, 32)),           # 64 chains over 144 MB of images
+    ([3000, 2000], Heads(16, 16, 32)),           # 64 chains over 97 MB of images
 ])
 def test_prefill_two_kernel_path(gpu, lens, heads):
     """Batches of at most 64 chains with a workspace: a first kernel prepares every
     chunk's T~, P and gates (all chunks at once) and the state pass copies them instead
     of recomputing them in each of a chain's 4 or 8 slices; split 8 ways, four consumer
     waves share each slice's chunk tokens.  Every value comes from the same operations in
-    the same order, so the results equal gdn_prefill's bit for bit (one kernel, except for
-    [130, 2100] and [3000, 2000], whose sequences average at least 1,024 tokens: gdn_prefill
-    runs those two kernels itself, in its own scratch); both match the oracle.  The
-    workspace starts as 0xFF bytes, so a chunk image that the first kernel did not write
-    would show."""
+    the same order, so the results equal one kernel's bit for bit (launched by the testing
+    entry point, which has no two-kernel path of its own), as do gdn_prefill's, whichever it
+    runs; both match the oracle.  The workspace starts as 0xFF bytes, so a chunk image that
+    the first kernel did not write would show."""
     say(f"prefill two-kernel path lens={lens} heads={heads}")
     p = workloads.prefill_inputs(lens, heads, seed=22, gate="slow", state_scale=0.5)
+    o0, s0, _ = _prefill_fault_injection(p, gpu, 0, 0)
     o1, s1 = _prefill_capi(p, gpu, workspace=False)
     o2, s2 = _prefill_capi(p, gpu, workspace=True)
+    assert torch.equal(o0, o2) and torch.equal(s0, s2), "workspace path differs from one kernel"
     assert torch.equal(o1, o2) and torch.equal(s1, s2), "workspace path differs from gdn_prefill"
     o_ref, s_ref = oracle_prefill(p)
     assert_close(host(o2), o_ref, OUT_RTOL, OUT_ATOL, "output")
@@ -400,8 +417,8 @@ def test_prefill_dropin_random_long_batches(gpu, seed):
     chains whose sequences average at least 1,024 tokens, images within its scratch):
     1-3 sequences of 1-2,000 tokens topped up to that average, random head layouts, gate
     regime, initial states and cu_seqlens dtype.  gdn_prefill equals
-    gdn_prefill_with_workspace bit for bit, both match the oracle, and no hand-off gives
-    up."""
+    gdn_prefill_with_workspace and one kernel bit for bit, all match the oracle, and no
+    hand-off gives up."""
     rng = np.random.default_rng(3000 + seed)
     hq, hk, hv = [(16, 16, 32), (8, 8, 16), (4, 8, 8), (2, 2, 4), (4, 4, 16)][int(rng.integers(0, 5))]
     n = min(int(rng.integers(1, 4)), 64 // hv)
@@ -418,9 +435,12 @@ def test_prefill_dropin_random_long_batches(gpu, seed):
                                  state_scale=0.5 if gate == "slow" else 0.05, with_state=with_state,
                                  cu_dtype=cu_dtype)
     binding.prefill_giveups(reset=True)
+    assert _dropin_windows(p) == (1, 0)
+    o0, s0, _ = _prefill_fault_injection(p, gpu, 0, 0)
     o1, s1 = _prefill_capi(p, gpu, workspace=False)
     o2, s2 = _prefill_capi(p, gpu, workspace=True)
     assert torch.equal(o1, o2) and torch.equal(s1, s2), "gdn_prefill differs from gdn_prefill_with_workspace"
+    assert torch.equal(o0, o1) and torch.equal(s0, s1), "gdn_prefill differs from one kernel"
     o_ref, s_ref = oracle_prefill(p)
     assert_close(host(o1), o_ref, OUT_RTOL, OUT_ATOL, "output")
     assert_close(host(s1), s_ref, STATE_RTOL, STATE_ATOL, "new_state")
@@ -434,11 +454,11 @@ def test_prefill_dropin_random_long_batches(gpu, seed):
 ])
 def test_prefill_prep_kernel_edges(gpu, lens, heads):
     """The prep kernel (a wave per chunk-head) where its indexing can go wrong: many
-    sequences, odd head counts, ragged and empty sequences.  Bit for bit gdn_prefill's
-    one kernel, and within tolerance of the oracle."""
+    sequences, odd head counts, ragged and empty sequences.  Bit for bit one kernel, and
+    within tolerance of the oracle."""
     say(f"prefill prep kernel edges lens={lens} heads={heads}")
     p = workloads.prefill_inputs(lens, heads, seed=92, gate="slow", state_scale=0.5)
-    o1, s1 = _prefill_capi(p, gpu, workspace=False)
+    o1, s1, _ = _prefill_fault_injection(p, gpu, 0, 0)
     o2, s2 = _prefill_capi(p, gpu, workspace=True)
     assert torch.equal(o1, o2) and torch.equal(s1, s2)
     o_ref, s_ref = oracle_prefill(p)
@@ -714,6 +734,7 @@ def test_prefill_dropin_scratch_path(gpu, in_place):
     gdn_prefill_with_workspace."""
     say(f"prefill drop-in scratch path, 2,500 tokens, in_place={in_place}")
     p = workloads.prefill_inputs([2500], seed=61, gate="slow", state_scale=0.5, cu_dtype=torch.int64)
+    assert _dropin_windows(p) == (1, 0)
     o_ref, s_ref = oracle_prefill(p)
     out, ns = run_prefill(p, gpu, in_place=in_place)
     out2, ns2 = run_prefill(p, gpu, in_place=False)
@@ -729,14 +750,15 @@ def test_prefill_dropin_scratch_path(gpu, in_place):
 
 
 def test_prefill_dropin_long_sequence(gpu):
-    """A 12,288-token sequence (32 v-heads: 118 MB of chunk images, more than 64 MiB, so
-    the state pass loads them two chunks ahead) runs two kernels in the drop-in's
-    scratch: against the oracle, and bit for bit equal to gdn_prefill_with_workspace."""
+    """A 12,288-token sequence (32 v-heads: 118 MB of chunk images, most of the drop-in's
+    scratch) runs two kernels there in one window: against the oracle, and bit for bit equal
+    to gdn_prefill_with_workspace."""
     say("prefill drop-in, one 12,288-token sequence")
     lib = _lib.load()
     p = workloads.prefill_inputs([12288], seed=62, gate="slow", state_scale=0.5)
     need = lib.gdn_prefill_workspace_size(1, 12288, 32)
     assert 64 << 20 < need <= _lib.GDN_PREFILL_DROPIN_SCRATCH_BYTES, need
+    assert _dropin_windows(p) == (1, 0)
     o_ref, s_ref = oracle_prefill(p)
     out, ns = run_prefill(p, gpu)
     o2, s2 = _prefill_capi(p, gpu, workspace=True)
@@ -746,25 +768,39 @@ def test_prefill_dropin_long_sequence(gpu):
     assert torch.equal(out, o2) and torch.equal(ns, s2)
 
 
-@pytest.mark.parametrize("lens,in_place", [
-    ([15001], True),           # one sequence, 32 chains: two windows
-    ([10500, 4700], False),    # 64 chains split 4 ways; one sequence ends in the first window
+@pytest.mark.parametrize("lens,heads,windows,state,cu_dtype", [
+    ([15001], Heads(16, 16, 32), 2, "in place", torch.int32),        # 32 chains, split 8 ways
+    ([10500, 4700], Heads(16, 16, 32), 3, "new", torch.int64),       # 64 chains split 4 ways; one ends first
+    ([28001], Heads(16, 16, 32), 3, None, torch.int32),              # no initial state
+    ([19001], Heads(12, 12, 24), 2, "new", torch.int64),             # 192 workgroups
+    ([0, 15000], Heads(16, 16, 32), 3, None, torch.int64),           # an empty sequence, zeroed once
+    ([9400, 0], Heads(24, 24, 24), 1, "in place", torch.int32),      # split 4 ways, only as offsets that overlap
+                                                                     # cannot come from two sequences
+    ([3000, 5900], Heads(16, 16, 48), 1, "new", torch.int64),        # split 2 ways, the same
+    ([8192, 8192], Heads(16, 16, 48), 0, "new", torch.int32),        # split 2 ways, beyond one window
+    ([30000], Heads(8, 8, 16), 0, None, torch.int32),                # windows would leave half the CUs idle
 ])
-def test_prefill_dropin_windows(gpu, lens, in_place):
+def test_prefill_dropin_windows(gpu, lens, heads, windows, state, cu_dtype):
     """Batches whose chunk images exceed the drop-in's scratch run in windows of the
-    sequences, the state carried from one to the next in new_state: against the oracle,
-    and bit for bit equal to gdn_prefill_with_workspace (one window)."""
-    say(f"prefill drop-in in windows, lens={lens} in_place={in_place}")
+    sequences, the state carried from one to the next in new_state: the expected number of
+    windows, within tolerance of the oracle, and bit for bit one kernel (and, where the batch
+    takes a workspace, gdn_prefill_with_workspace, one window)."""
+    say(f"prefill drop-in in windows, lens={lens} heads={heads} state={state}")
     lib = _lib.load()
     T, N = sum(lens), len(lens)
-    assert ((T + 63) // 64 + N - 1) * 32 * 19200 > _lib.GDN_PREFILL_DROPIN_SCRATCH_BYTES
-    assert lib.gdn_prefill_workspace_size(N, T, 32) > 0
-    p = workloads.prefill_inputs(lens, seed=64, gate="slow", state_scale=0.5)
-    o2, s2 = _prefill_capi(p, gpu, workspace=True)
+    assert N * ((T + 63) // 64) * heads.hv * 19200 > _lib.GDN_PREFILL_DROPIN_SCRATCH_BYTES
+    p = workloads.prefill_inputs(lens, heads, seed=64, gate="slow", state_scale=0.5, with_state=state is not None,
+                                 cu_dtype=cu_dtype)
+    assert _dropin_windows(p) == (windows, int(windows > 0 and heads.hv * N > 64))
+    o1, s1, aborts = _prefill_fault_injection(p, gpu, 0, 0)
     o_ref, s_ref = oracle_prefill(p)
-    out, ns = run_prefill(p, gpu, in_place=in_place)
+    out, ns = run_prefill(p, gpu, in_place=state == "in place")
     torch.cuda.synchronize()
-    assert torch.equal(out, o2) and torch.equal(ns, s2)
+    assert int(aborts.item()) == 0
+    assert torch.equal(out, o1) and torch.equal(ns, s1)
+    if lib.gdn_prefill_workspace_size(N, T, heads.hv) > 0:
+        o2, s2 = _prefill_capi(p, gpu, workspace=True)
+        assert torch.equal(out, o2) and torch.equal(ns, s2)
     assert_close(host(out), o_ref, OUT_RTOL, OUT_ATOL, "output")
     assert_close(host(ns), s_ref, STATE_RTOL, STATE_ATOL, "new_state")
 
@@ -778,11 +814,12 @@ def test_prefill_dropin_windows(gpu, lens, in_place):
     ([639], Heads(16, 16, 32), False),
 ])
 def test_prefill_dropin_rule_edges(gpu, lens, heads, two_kernels):
-    """Around the lines of the drop-in's choice between one kernel and two: bit for bit the
-    one kernel (launched through the testing entry point with its hooks off), and within
-    tolerance of the oracle.  (two_kernels: which side of the line; the results do not tell.)"""
+    """Around the lines of the drop-in's choice between one kernel and two: the expected side
+    of the line, bit for bit the one kernel (launched through the testing entry point with its
+    hooks off), and within tolerance of the oracle."""
     say(f"prefill drop-in rule lens={lens} heads={heads} two_kernels={two_kernels}")
     p = workloads.prefill_inputs(lens, heads, seed=65, gate="slow", state_scale=0.5)
+    assert _dropin_windows(p)[0] == int(two_kernels)
     o1, s1, aborts = _prefill_fault_injection(p, gpu, 0, 0)
     o2, s2 = run_prefill(p, gpu)
     torch.cuda.synchronize()
