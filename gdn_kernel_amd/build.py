@@ -30,7 +30,6 @@ HIPCC_FLAGS = [
     "-fPIC",
     "-shared",
     "-Wall",
-    "-Wno-unused-function",
     # No packed-fp32 VALU ops in device code (v_pk_{add,mul,fma}_f32).
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]

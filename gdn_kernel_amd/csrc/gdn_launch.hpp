@@ -79,9 +79,7 @@ hipError_t decode_pool_conflicts(uint64_t* count, bool reset);
 // chains on the current device (the grid times the workgroup size of the variant
 // the launcher picks).
 int64_t prefill_work_items(int64_t chains);
-// `done`, if not null, is recorded when the launch's last kernel completes (the
-// two-kernel path only: callers that pass it have set args.tiles).
-hipError_t launch_prefill(const PrefillArgs& args, hipStream_t stream, hipEvent_t done = nullptr);
+hipError_t launch_prefill(const PrefillArgs& args, hipStream_t stream);
 
 // Bytes of the per-device scratch array of gdn_prefill_no_alloc, and its address
 // on the current device (looked up on the first call per device).

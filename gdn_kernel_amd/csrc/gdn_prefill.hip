@@ -502,15 +502,6 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
   return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-x * 1.4426950408889634f));
 }
 
-// Sum over the four 16-lane rows of a wavefront (lanes j, j+16, j+32, j+48):
-// the row swaps pair rows (0,1), (2,3), then the two halves.
-__device__ __forceinline__ float sum_rows(float x) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // Orders this wave's LDS writes before its later LDS reads by other lanes.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -579,9 +570,9 @@ __device__ __forceinline__ void signal_count(Smem& sm, int which, int lane) {
 // can cause), it raises kAbort, and all later waits return at once, so the
 // workgroup still finishes instead of hanging.  The wave that gives up adds 1 to
 // gdn_prefill_giveup_count (a global atomic from one lane), and the workgroup
-// writes NaN to every output element and state element it owns, so wrong results never look valid.  Production kernels give
-// up after kSpinLimit polls; kernels built with the hooks after sm.spin_limit
-// polls, also counting each give-up in sm.aborts if set.
+// writes NaN to every output element and state element it owns, so wrong results never
+// look valid.  Production kernels give up after kSpinLimit polls; kernels built with the
+// hooks after sm.spin_limit polls, also counting each give-up in sm.aborts if set.
 template <bool kHooks, class Smem>
 __device__ __forceinline__ void wait_count(Smem& sm, int which, int target) {
   if (__hip_atomic_load(&sm.sync[which], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < target) {
@@ -1018,13 +1009,6 @@ __device__ __forceinline__ void stage_kq(const ChunkBufs& cb, const ProducerPref
     *reinterpret_cast<uint2*>(cb.Q + pa) = uint2{f.q[it].x, f.q[it].y};
     *reinterpret_cast<uint2*>(cb.Q + pb) = uint2{f.q[it].z, f.q[it].w};
   }
-}
-
-// Step 1 with the chunk's gates formed in place (first wave).
-__device__ __forceinline__ void stage_kq_gates(const ChunkBufs& cb, const ProducerPrefetch& f, int pt, int pw, int lane,
-                                               int clen, float neg_decay, float dt_bias) {
-  stage_kq(cb, f, pt);
-  if (pw == 0) store_gates(cb, chunk_gates(f, lane, clen, neg_decay, dt_bias), lane);
 }
 
 // Unit g of a chunk's gates (beta, e^gamma, e^{gamma_last - gamma}; 16 units each),
@@ -1838,10 +1822,8 @@ __global__ __launch_bounds__(V::NTHREADS) void gdn_prefill_kernel(PrefillArgs p)
   const int tid = threadIdx.x;
   const int lane0 = tid & 63;
   const int hw = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Role index.  Waves are dealt to the four SIMDs round-robin.  In the loader
-  // variant with one consumer, the consumer takes hardware wave 3, a SIMD to itself,
-  // and two (mostly idle) loaders share SIMD 0: config 3 174 -> 170 us.  Elsewhere
-  // the natural order measured as fast or faster (two consumers on SIMDs of their
+  // Role index.  Waves are dealt to the four SIMDs round-robin.  With four producers or
+  // loaders the natural order measured as fast or faster (two consumers on SIMDs of their
   // own: +1.5%; the producer variant's solve wave sharing a SIMD: +7%).
   // With seven producers (beside one consumer) the consumer keeps hardware wave 0 and
   // shares its SIMD with the producer that has least to do (wave 0, the solve): hardware
@@ -1852,8 +1834,7 @@ __global__ __launch_bounds__(V::NTHREADS) void gdn_prefill_kernel(PrefillArgs p)
   // second consumer with the right off-diagonal wave, or the two off-diagonal waves).
   const int wave = V::NP == 7   ? (hw == 0 ? 0 : 1 + ((0x6540321 >> (4 * (hw - 1))) & 15))
                    : V::NP == 6 ? (hw < 2 ? hw : 2 + ((0x415032 >> (4 * (hw - 2))) & 15))
-                   : !(V::kLoad && NCW == 1) ? hw
-                   : hw == 3 ? 0 : hw < 3 ? hw + 1 : hw;
+                                : hw;
 
   const int bid = blockIdx.x;
   // Workgroups are dealt to the 8 XCDs round-robin.  F == 1: blocks b and b + 8 of
@@ -2509,7 +2490,6 @@ __device__ __forceinline__ void state_consumer(Smem& sm, const PrefillArgs& p, i
         const uint2 k0 = read_tr(kp), k1 = read_tr(kp + 16 * KSTR);
         kt[j][js] = uint4{k0.x, k0.y, k1.x, k1.y};
       }
-    // What the next chunk's retrieve and Y take besides the state.
     signal_count(sm, kChunkRead, lane);  // buffers of this chunk no longer read
     __builtin_amdgcn_sched_barrier(0);
 
@@ -3250,10 +3230,10 @@ hipError_t launch_two_kernels(const PrefillArgs& a, hipStream_t stream, int64_t 
 }
 }  // namespace
 
-hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream, hipEvent_t done) {
+hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
   const int F = split_factor(int64_t(a.N) * a.Hv);
   if (a.tiles != nullptr && prefill_workspace_bytes(a.N, a.T, a.Hv) > 0)
-    return launch_two_kernels(a, stream, a.N * ((a.T + C - 1) / C), done);
+    return launch_two_kernels(a, stream, a.N * ((a.T + C - 1) / C), nullptr);
   if (has_hooks(a)) {
     if (persistent_batch(a)) return launch_persistent<PersistVariant<true>>(a, stream);
     switch (F) {
