@@ -250,7 +250,8 @@ def prefill_kernel(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, outp
 
 def prefill_workspace_bytes(num_seqs: int, total_tokens: int, num_v_heads: int, device=None) -> int:
     """Bytes of workspace ``prefill_kernel_with_workspace`` uses for a batch of this size on
-    ``device`` (gdn_prefill_workspace_size); 0 when the batch runs one kernel anyway."""
+    ``device`` (gdn_prefill_workspace_size); 0 for a batch that takes none: give it to
+    ``prefill_kernel``."""
     lib = _lib.load()
     dev = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     with _on_device(dev):
@@ -263,8 +264,9 @@ def prefill_kernel_with_workspace(q, k, v, state, A_log, a, dt_bias, b, cu_seqle
     no reference counterpart): batches of few (sequence, v-head) chains then prepare
     each chunk once in a first kernel, for the same results bit for bit.  ``workspace``
     is a contiguous uint8 tensor of at least ``prefill_workspace_bytes(N, T, Hv)`` bytes
-    on the same device (or None: ``prefill_kernel``); launches that may overlap must
-    not share one."""
+    on the same device; launches that may overlap must not share one.  With None, or for
+    a batch that takes no workspace, it runs one kernel (``prefill_kernel`` instead runs
+    batches of few long sequences as two kernels in the library's scratch)."""
     rc = _lib.native().prefill_with_workspace(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale,
                                               output, new_state, workspace)
     if rc is not None:

@@ -46,7 +46,7 @@ struct PrefillArgs {
   int ready_chunks;         // > 0: producers signal "chunk ready" only for chunks < ready_chunks
   unsigned* aborts;         // non-null: +1 (device atomic) each time a wait gives up
   // Two-kernel path: workspace of prefill_workspace_bytes(...) bytes for the
-  // prepared T~/P tiles; null (or a batch that the single kernel serves) => one kernel.
+  // prepared T~/P tiles; null (or a batch that takes no workspace) => one kernel.
   uint16_t* tiles;
   // Set by the launcher of the two-kernel path: the most chunks a launch with valid offsets
   // covers, and the launch's window of each sequence (win_tokens = 0: all of it).
@@ -55,8 +55,7 @@ struct PrefillArgs {
 };
 
 // Workspace bytes of the two-kernel prefill path for these sizes on the current
-// device, or 0 when the single kernel serves them (many chains, or a workspace
-// above the cap).
+// device, or 0 for batches that take no workspace (many chains, or one above the cap).
 int64_t prefill_workspace_bytes(int N, int64_t T, int Hv);
 
 // Decode launch shapes (rows per wave x waves per workgroup x nontemporal state

@@ -24,10 +24,13 @@
 // chains are split so that every CU gets a workgroup (with F = 8 and F = 4 one or
 // two 16-row consumers beside seven or six pipelined producers, since the chunk
 // preparation, repeated in every slice, sets the pace).
-// When the caller provides
-// a workspace, batches split 4 or 8 ways run in two kernels instead: a prep kernel
-// prepares every chunk once (all chunks in parallel), and the state pass's loader
-// waves copy its T~/P tiles where the producers would have computed them.
+//
+// Batches of few chains can run in two kernels instead: a prep kernel prepares every
+// chunk once (all chunks in parallel), and a state pass takes its T~, P and gates from
+// memory.  Split 8 ways the state pass is gdn_prefill_state_kernel; split 4 or 2 ways it
+// is a variant of the kernel above, whose loader waves copy the tiles where the producers
+// would have computed them.  Split 4 and 8 ways the path runs in a caller's workspace or
+// in the library's scratch, split 2 ways in the drop-in's scratch only (dropin_route).
 //
 // Per chunk (positions >= clen are zero-padded: K = Q = V = 0, beta = 0 and
 // log-gate 0, as kernel_prefill.cu:102-114, 125-132 pads them):
@@ -1437,7 +1440,7 @@ __device__ __forceinline__ void producer_loop_split(PrefillSmem& sm, const Prefi
 // latency overlaps the waits for the consumers.
 // V goes two chunks ahead in every variant (two register sets): the prep kernel does
 // not read V, so with inputs that the caches do not hold its loads come from HBM
-// (config 3 with four rotating input sets: 142.5 -> 132.0 us, unchanged with one).
+// (one 4,096-token sequence, four rotating input sets: 142.5 -> 132.0 us, unchanged with one).
 template <class V>
 __device__ __forceinline__ void loader_loop(PrefillSmem& sm, const PrefillArgs& p, const u32x4* tiles, int64_t s0,
                                             int64_t s1, int nchunks, int h, int hq, int hk, int row0, int pw,
@@ -2541,7 +2544,7 @@ __device__ __forceinline__ void state_consumer(Smem& sm, const PrefillArgs& p, i
 
 // Workgroup b handles slice f (16 state rows) of chain `chain` (rank-major, v-head minor),
 // placed as in gdn_prefill_kernel with F = 8: the slices of a GQA pair of chains share an
-// XCD.  Waves 0-3 are consumers, 4-7 loaders.
+// XCD.  Waves 0-3 are consumers, 4-7 helpers.
 constexpr int kStateSlices = 8;
 template <bool HOOKS>
 __global__ __launch_bounds__(512) void gdn_prefill_state_kernel(PrefillArgs p) {
@@ -2650,11 +2653,15 @@ __device__ __forceinline__ Pair2 get_block(const uint16_t (&blk)[2][256], int la
 // registers (an N tile's accumulator layout is the A operand the off-diagonal solve takes),
 // the tiles (I, J) of N and P share their decays, and every fragment of the image leaves
 // the registers as a linear 16-byte store.  A chunk-head is a chain of dependent steps
-// (about 9k cycles of arithmetic and 5k of first loads), so what counts is how many are in
-// flight: 12 waves a CU, no barriers.  One 4,096-token sequence at 32 v-heads (2,048
-// chunk-heads, 72 MB of K, Q and images, inputs from HBM) takes 20.6 us, 12,288 tokens
-// 51.7; a workgroup of four waves per run of chunks, handing over through the LDS (two
-// workgroups a CU), took 26.9 and about 80.
+// (about 9k cycles of arithmetic and 5k of first loads), so a small batch takes that long
+// whatever its size (32 v-heads, inputs cached: 640 tokens, 320 chunk-heads, 8.9 us, 1,024
+// tokens 9.4), and what counts is how many are in flight: 12 waves a CU, no barriers.
+// Larger batches move towards the memory's pace: 2,048 tokens 14.2, 4,096 22.2, 8,192 37.0,
+// 12,288 50.8, the last 145 MB of K, Q and images at 5.1 TB/s, where a device copy reaches
+// 5.3 (a sixth of the tile bytes are the zeros of fragments (0, 0) and (2, 1)).  A
+// workgroup of four waves per run of chunks, handing over through the LDS (two workgroups a
+// CU), took 26.9 us at 4,096 tokens with inputs from HBM against 20.6, and about 80 at
+// 12,288 against 51.7.
 constexpr int kPrepWaves = 2;
 __global__ __launch_bounds__(64 * kPrepWaves, 2) void gdn_prefill_prep_kernel(PrefillArgs p) {
   __shared__ PrepSmem smem[kPrepWaves];
@@ -3162,9 +3169,10 @@ constexpr int64_t kMaxWorkspaceBytes = int64_t(2) << 30;
 // Batches split 4 or 8 ways repeat the producer work in every slice of a chain and
 // are bound by it; the two-kernel path prepares each chunk once, all chunks in
 // parallel, and its state pass (no producer code: 16-row consumers fit in the
-// registers) runs at the consumers' pace.  Batches split 2 ways lose more to the
-// extra pass than they gain, and unsplit ones keep producers and consumers busy
-// on the same CUs.
+// registers) runs at the consumers' pace.  Batches split 2 ways take no workspace
+// (some of them gain from two kernels all the same: dropin_route), and unsplit ones
+// keep producers and consumers busy on the same CUs.  The size holds the chunks of any
+// offsets, also of malformed ones that overlap: N ceil(T / C) a v-head.
 int64_t prefill_workspace_bytes(int N, int64_t T, int Hv) {
   if (N <= 0 || Hv <= 0 || T <= 0 || split_factor(int64_t(N) * Hv) < 4) return 0;
   const int64_t images = int64_t(N) * ((T + C - 1) / C) * Hv;

@@ -110,7 +110,7 @@ int gdn_decode_check(const gdn_bf16* q, const gdn_bf16* k, const gdn_bf16* v,
  *   state_indices [B] int32 device array; an index outside [0, pool_slots)
  *                 marks a padding row: its output is zero and no slot is touched.
  * A slot that two or more valid rows name is a conflict: updating it from both rows
- * would race.  The kernel detects it on the device before it touches any state
+ * would race.  The kernel detects it on the device before it writes any state
  * (each row's workgroups scan the B indices) and skips every such row like a padding
  * row (zero output, slot untouched); gdn_decode_pool_conflicts counts the skipped
  * rows.  Other arguments as gdn_decode.
@@ -167,7 +167,7 @@ int64_t gdn_static_device_bytes(void);
  * scratch array the library holds on each device (GDN_PREFILL_DROPIN_SCRATCH_BYTES,
  * its own, not gdn_prefill_no_alloc's).  The chunk images take 19,200 bytes per 64-token
  * chunk and v-head (one sequence with 32 v-heads: up to 13,952 tokens at a time;
- * BASELINE's 4,096-token sequence needs 37.5 MiB); one or two sequences that need more and
+ * a 4,096-token one needs 37.5 MiB); one or two sequences that need more and
  * have 24 to 32 or 48 to 64 chains (a workgroup on three quarters of the CUs) run in windows,
  * the state carried from one to the next, and others that do not fit (more sequences: with
  * any offsets, num_seqs ceil(total_tokens / 64) chunks) run one kernel.  The results are the
@@ -207,14 +207,17 @@ int gdn_prefill_check(const gdn_bf16* q, const gdn_bf16* k, const gdn_bf16* v,
  * preparation runs once per chunk in a first kernel, for all chunks in
  * parallel, and the state pass only copies it.
  *   gdn_prefill_workspace_size: bytes this path needs for num_seqs sequences,
- *     total_tokens tokens and num_v_heads v-heads on the current device;
- *     0 when gdn_prefill serves the batch with one kernel anyway (more chains,
- *     or more than 2 GiB of workspace).  Touches no device memory.
+ *     total_tokens tokens and num_v_heads v-heads on the current device, whatever
+ *     their offsets (num_seqs ceil(total_tokens / 64) chunk images a v-head); 0 for
+ *     batches that take no workspace (more chains, or more than 2 GiB of it).  Touches
+ *     no device memory.
  *   gdn_prefill_with_workspace: gdn_prefill's arguments plus the workspace
  *     (16-byte aligned, at least the size above, and not shared with a launch
- *     that may run concurrently).  A NULL workspace, or a batch whose size is 0,
- *     runs gdn_prefill.  The results equal gdn_prefill's bit for bit (the same
- *     code prepares the chunks).
+ *     that may run concurrently).  With a NULL workspace, or for a batch whose size is
+ *     0, it runs one kernel and does not use the library's scratch: a caller without a
+ *     workspace calls gdn_prefill, which also runs two kernels for some batches that
+ *     take none (65 to 96 chains of long sequences).  The results equal gdn_prefill's
+ *     bit for bit (the same code prepares the chunks).
  */
 int64_t gdn_prefill_workspace_size(int64_t num_seqs, int64_t total_tokens,
                                    int32_t num_v_heads);
@@ -237,8 +240,8 @@ int gdn_prefill_with_workspace(const gdn_bf16* q, const gdn_bf16* k, const gdn_b
  * (GDN_PREFILL_NO_ALLOC_SCRATCH_BYTES, allocated when the library's code is
  * loaded onto the device and kept until the process ends).  Nothing is allocated
  * per call.  A batch whose images need more than that (gdn_prefill_workspace_size
- * above it) returns GDN_ERR_INVALID_ARGUMENT; batches that gdn_prefill serves with
- * one kernel need no scratch.  Every call on a device shares that device's
+ * above it) returns GDN_ERR_INVALID_ARGUMENT; batches whose size is 0 run one kernel
+ * and need no scratch.  Every call on a device shares that device's
  * scratch.  Calls on streams that are not being captured are ordered on the device
  * like gdn_prefill's (their own mutex and event), so eager calls on any streams stay
  * correct.  A call captured into a graph cannot wait for that event: its replays

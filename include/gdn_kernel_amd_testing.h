@@ -28,7 +28,8 @@ extern "C" {
  *                0: no limit.  Must be >= 0.
  *   aborts       device uint32 counter (or NULL): incremented once by each
  *                wavefront whose wait gives up.  The caller clears it.
- * With spin_limit = ready_chunks = 0 and aborts = NULL this is gdn_prefill.
+ * It always runs one kernel; with spin_limit = ready_chunks = 0 and aborts = NULL, the one
+ * that gdn_prefill runs where it does not run two.
  */
 int gdn_prefill_fault_injection(const gdn_bf16* q, const gdn_bf16* k, const gdn_bf16* v,
                                 const float* state, const float* A_log, const gdn_bf16* a,
