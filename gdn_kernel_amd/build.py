@@ -106,7 +106,11 @@ def build_native(verbose: bool = False) -> Path:
     out = native_path()
     tmp = out.with_name(out.name + ".tmp")
     cxx = os.environ.get("CXX") or shutil.which("g++") or "c++"
-    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+    # NDEBUG, as torch itself is built: without it the headers bring a thread-local counter,
+    # and loading a module with a TLS segment that the thread never reads puts every later
+    # thread-local access of the thread on glibc's slow path: a torch view took 0.70 us
+    # instead of 0.56, in calls that have nothing to do with this module.
+    cmd = [cxx, "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-Wall",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
            f'-DGDN_NATIVE_TORCH="{torch.__version__}"', f'-DGDN_NATIVE_LIBRARY="{source_digest()}"',
            f'-DGDN_NATIVE_BUILD_ID="{native_digest()}"',

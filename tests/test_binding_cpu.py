@@ -1,6 +1,7 @@
 """CPU tests of the Python binding's argument checks and of the workload
 generators (no GPU; nothing is launched)."""
 import math
+import struct
 import sys
 
 import numpy as np
@@ -92,6 +93,17 @@ def test_native_module_is_built_from_these_sources():
     assert _native.build_id == build.native_digest()
     assert _native.library_build_id == build.source_digest() == _lib.load().gdn_build_id().decode()
     assert _native.torch_version == str(torch.__version__)
+
+
+def test_native_module_has_no_tls_segment():
+    """A TLS segment in the module would slow down every torch call of the thread that
+    imports it (see build_native)."""
+    from gdn_kernel_amd import build
+    elf = build.native_path().read_bytes()
+    assert elf[:6] == b"\x7fELF\x02\x01"
+    at, size, count = (struct.unpack_from("<Q", elf, 0x20)[0], *struct.unpack_from("<HH", elf, 0x36))
+    types = [struct.unpack_from("<I", elf, at + i * size)[0] for i in range(count)]
+    assert 1 in types and 7 not in types            # PT_LOAD, no PT_TLS
 
 
 @pytest.mark.parametrize("cxx", ["absent", "failing"])
